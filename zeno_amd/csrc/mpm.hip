@@ -308,6 +308,17 @@ __global__ void __launch_bounds__(kThreads) k_gather_state(State src, int64_t sr
     }
 }
 
+// Inclusive sum over the wave's lanes by DPP row shifts and broadcasts.
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
 // ------------------------------------------------------------------ P2G
 constexpr int kP2GThreads = 192;             // 3 waves: wave g handles the stencil x-offset ox = g in phase B
 constexpr int kP2GRounds = 2;                // phase A rounds of 192 particles
@@ -896,6 +907,202 @@ k_p2g(State A, Partition P, Lattice L, const DevMaterial *mats,
             }
         }
         if (!FLUSH) p2g_tiles_out(acc, s_pl, s_task, tb, true);
+    }
+    if (mismatch) atomicOr(&st->bin_mismatch, 1u);
+}
+
+// P2G of few parts: k_p2g's sums, bit for bit, with nine waves a part, for launches whose parts do
+// not fill the chip, where a part's chain of dependent steps is the launch's time.  Thread =
+// particle for the payload (576 a chunk, so a block at 8 per cell needs one; every field loaded at
+// the start); then wave = (x-offset, y-offset), lane = cell: three nodes x 4 channels a thread
+// instead of nine.  A node's additions are those of k_p2g in its order: the particles of a cell one
+// after another, across the chunks in registers; the cells' sums into the x-offset's tile by
+// (oy, oz), where one wave holds all of an (ox, oy), so only the three oy are a barrier apart.
+// Launches of 35 and 180 parts: 17.9 -> 12.9 and 17.8 -> 13.7 us; 366 parts (more than the CUs):
+// 14.7 -> 16.6, 576: 16.4 -> 26, as the threads' weights are formed nine times, not three.
+constexpr int kWideThreads = 576;
+constexpr int kWideWaves = kWideThreads / 64;
+template <int MODE, bool PP>
+__global__ void __launch_bounds__(kWideThreads)
+k_p2g_wide(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t sig_stride,
+           float *tiles, DevStatus *st, AdjScatter adj) {
+    __shared__ float s_pl[kPL * kWideThreads];
+    __shared__ float4 s_tile[3 * kTileNodes];
+    __shared__ uint32_t s_wcnt[kWideWaves][64];
+
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int ox = w / 3, oy = w % 3;
+    const XWeight xk = xweight_of(ox), yk = xweight_of(oy);
+    const float fox = (float)ox;
+    const uint32_t nblocks = P.counts[0], nx = P.counts[2];
+    const PartView V = part_view(P, L.part_shift);
+    bool mismatch = false;
+    for (uint32_t j = blockIdx.x; j < nblocks + nx; j += gridDim.x) {
+        const PartRef pr = part_ref(V, j, nblocks);
+        const uint32_t b = pr.b, ps = pr.lo, pe = pr.hi;
+        const SceneParams sc = scene_params(L, L.nscenes == 1 ? 0u : P.pblk_scene[b]);
+        const float dx = sc.dx, dxinv = sc.dxinv;
+        const float sdt = -sc.dt * sc.Dinv;
+        int lbx, lby, lbz;
+        lattice_coords(sc, P.pblk_lat[b], lbx, lby, lbz);
+        const int bc[3] = {(lbx + L.origin) * 4, (lby + L.origin) * 4, (lbz + L.origin) * 4};
+        for (int k = t; k < 3 * kTileNodes; k += kWideThreads) s_tile[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float acc[12];
+#pragma unroll
+        for (int q = 0; q < 12; ++q) acc[q] = 0.0f;
+        for (uint32_t c0 = ps; c0 < pe; c0 += kWideThreads) {
+            const uint32_t i = min(c0 + (uint32_t)t, pe - 1u);
+            const bool valid = c0 + (uint32_t)t < pe;
+            // ---- fields, cell and stable slot
+            const TileRun run = tile_run(A.ch, c0);
+            const uint32_t off = run_off(run, i);
+            float xp[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) xp[k] = run_chan(run, off, k);
+            P2GIn in;
+            if (MODE != kP2GAdjoint) p2g_load(A, run, off, in, PP);
+            float fr[3];
+            int lc[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float X = xp[k] * dxinv;
+                const int base = cell_floor(X);
+                fr[k] = X - (float)base;
+                lc[k] = base - bc[k];
+                mismatch |= valid && (lc[k] < 0 || lc[k] > 3);
+                lc[k] = clamp03(lc[k]);
+            }
+            const uint32_t cell = (uint32_t)((lc[0] * 4 + lc[1]) * 4 + lc[2]);
+            const uint64_t match = same_key_lanes<6>(cell, valid);
+            const uint32_t rank = count_below(match);
+            s_wcnt[w][lane] = 0u;
+            wave_lds_order();
+            if (valid && rank == 0u) s_wcnt[w][cell] = (uint32_t)__popcll(match);
+            __syncthreads();
+            uint32_t tot = 0u, before = 0u;
+#pragma unroll
+            for (int k = 0; k < kWideWaves; ++k) {
+                const uint32_t c = s_wcnt[k][lane];
+                tot += c;
+                before += k < w ? c : 0u;
+            }
+            const uint32_t end = wave_scan_u32(tot), start = end - tot;
+            const uint32_t slot = (uint32_t)__shfl((int)(start + before), (int)cell, 64) + rank;
+            // ---- payload in cell order (k_p2g's)
+            if (valid) {
+                float *pl = s_pl + slot;
+                if (MODE == kP2GAdjoint) {
+                    const float fdx[3] = {fr[0] * dx, fr[1] * dx, fr[2] * dx};
+                    pl[0] = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) pl[(1 + k) * kWideThreads] = fr[k];
+#pragma unroll
+                    for (int rr = 0; rr < 3; ++rr) {
+                        float Br[3];
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) Br[c] = adj.B[(3 * rr + c) * adj.stride + i];
+                        pl[(4 + rr) * kWideThreads] =
+                            adj.a[rr * adj.stride + i] - (Br[0] * fdx[0] + Br[1] * fdx[1] + Br[2] * fdx[2]);
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) pl[(7 + 3 * rr + c) * kWideThreads] = Br[c] * dx;
+                    }
+                } else if (MODE == kP2GFlipStress) {
+                    p2g_payload_flip_stress<kWideThreads>(in, i, mats, sig, sig_stride, dx, sc.dt, fr, pl);
+                } else {
+                    p2g_payload<kWideThreads, MODE == kP2GMomentum       ? 1
+                                              : MODE == kP2GStress       ? 2
+                                              : MODE == kP2GFlipMomentum ? 3
+                                                                         : 0>(in, i, mats, sig, sig_stride, dx, sdt,
+                                                                              fr, pl);
+                }
+            }
+            __syncthreads();
+            // ---- the cell's particles onto the nodes (ox, oy, 0 .. 2)
+            for (uint32_t s = start; s < end; ++s) {
+                float wz[3];
+                if (MODE == kP2GFlipStress) {  // as p2g_accumulate_grad
+                    float f[3], S[9], wx[3], wy[3];
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) f[q] = s_pl[(1 + q) * kWideThreads + s];
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) S[q] = s_pl[(4 + q) * kWideThreads + s];
+                    bspline_w(f[0], wx);
+                    bspline_w(f[1], wy);
+                    bspline_w(f[2], wz);
+                    const float wxo = ox == 0 ? wx[0] : (ox == 1 ? wx[1] : wx[2]);
+                    const float wyo = oy == 0 ? wy[0] : (oy == 1 ? wy[1] : wy[2]);
+                    const float dwxo = ox == 0 ? f[0] - 1.5f : (ox == 1 ? 2.0f * (1.0f - f[0]) : f[0] - 0.5f);
+                    const float dwyo = oy == 0 ? f[1] - 1.5f : (oy == 1 ? 2.0f * (1.0f - f[1]) : f[1] - 0.5f);
+                    const float dwz[3] = {f[2] - 1.5f, 2.0f * (1.0f - f[2]), f[2] - 0.5f};
+#pragma unroll
+                    for (int oz = 0; oz < 3; ++oz) {
+                        const float W = wxo * wyo * wz[oz];
+                        const float g[3] = {dwxo * wyo * wz[oz], wxo * dwyo * wz[oz], wxo * wyo * dwz[oz]};
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) {
+                            const float val = S[3 * r] * g[0] + S[3 * r + 1] * g[1] + S[3 * r + 2] * g[2];
+                            acc[4 * oz + 1 + r] = fmaf(W, val, acc[4 * oz + 1 + r]);
+                        }
+                    }
+                } else {  // as p2g_accumulate
+                    const float m = s_pl[s];
+                    float t3[3], bd[9];
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) bd[q] = s_pl[(7 + q) * kWideThreads + s];
+                    const float wxo = xweight(xk, s_pl[1 * kWideThreads + s]);
+                    const float wxy = wxo * xweight(yk, s_pl[2 * kWideThreads + s]);
+                    bspline_w(s_pl[3 * kWideThreads + s], wz);
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) {
+                        t3[r] = fmaf(fox, bd[3 * r], s_pl[(4 + r) * kWideThreads + s]);
+                        if (oy > 0) t3[r] += bd[3 * r + 1];
+                        if (oy > 1) t3[r] += bd[3 * r + 1];
+                    }
+#pragma unroll
+                    for (int oz = 0; oz < 3; ++oz) {
+                        const float W = wxy * wz[oz];
+                        acc[4 * oz] = fmaf(W, m, acc[4 * oz]);
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) {
+                            acc[4 * oz + 1 + r] = fmaf(W, t3[r], acc[4 * oz + 1 + r]);
+                            t3[r] += bd[3 * r + 2];
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        // ---- registers -> the x-offset's tile, one y-offset after another
+        float4 *col = s_tile + ox * kTileNodes + (((lane >> 4) + ox) * kTileSide + ((lane >> 2) & 3) + oy) * kTileSide +
+                      (lane & 3);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            if (oy == q) {
+#pragma unroll
+                for (int oz = 0; oz < 3; ++oz) {
+                    float4 v = col[oz];
+                    v.x += acc[4 * oz];
+                    v.y += acc[4 * oz + 1];
+                    v.z += acc[4 * oz + 2];
+                    v.w += acc[4 * oz + 3];
+                    col[oz] = v;
+                    wave_lds_order();
+                }
+            }
+            __syncthreads();
+        }
+        // ---- the three tiles in a fixed order -> HBM
+        float *tb = tiles + (int64_t)pr.p * (4 * kTileNodes);
+        if (t < kTileNodes) {
+            const float4 a0 = s_tile[t], a1 = s_tile[kTileNodes + t], a2 = s_tile[2 * kTileNodes + t];
+            const int slot = tile_slot_of(t);
+            tb[slot] = (a0.x + a1.x) + a2.x;
+            tb[kTileNodes + slot] = (a0.y + a1.y) + a2.y;
+            tb[2 * kTileNodes + slot] = (a0.z + a1.z) + a2.z;
+            tb[3 * kTileNodes + slot] = (a0.w + a1.w) + a2.w;
+        }
+        __syncthreads();
     }
     if (mismatch) atomicOr(&st->bin_mismatch, 1u);
 }
@@ -2890,16 +3097,30 @@ void launch_stress(State A, int64_t n, Lattice L, const DevMaterial *mats, float
         hipLaunchKernelGGL(k_stress<false>, dim3(grid_for(n, 2048)), dim3(kThreads), 0, s, A, n, L, mats, sig, stride);
 }
 
-// k_p2g<MODE> with or without the particles' own mass and volume (L.pp_mass)
+// P2G over `units` parts, the host's estimate (the count + 25 % + 64): k_p2g_wide while the count is
+// at most the chip's 256 CUs, where its shorter chain is the launch's time (figures at the kernel),
+// k_p2g above.  The two give the same bits.
+constexpr int64_t kWideMaxUnits = 384;
 template <int MODE>
-void launch_p2g_mode(dim3 g, hipStream_t s, State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig,
-                     int64_t stride, float *tiles, DevStatus *st, AdjScatter adj, uint32_t skip_upto) {
-    if (L.pp_mass)
-        hipLaunchKernelGGL((k_p2g<MODE, true>), g, dim3(kP2GThreads), 0, s, A, P, L, mats, sig, stride, tiles, st, adj,
-                           skip_upto);
-    else
+void launch_p2g_mode(int64_t units, hipStream_t s, State A, Partition P, Lattice L, const DevMaterial *mats,
+                     const float *sig, int64_t stride, float *tiles, DevStatus *st, AdjScatter adj,
+                     uint32_t skip_upto) {
+    const dim3 g(persistent_grid(units, 1, 1 << 20));
+    constexpr bool CAN_PP = MODE != kP2GAdjoint;
+    if (skip_upto == 0u && units <= kWideMaxUnits) {
+        if (CAN_PP && L.pp_mass)
+            hipLaunchKernelGGL((k_p2g_wide<MODE, CAN_PP>), g, dim3(kWideThreads), 0, s, A, P, L, mats, sig, stride,
+                               tiles, st, adj);
+        else
+            hipLaunchKernelGGL((k_p2g_wide<MODE, false>), g, dim3(kWideThreads), 0, s, A, P, L, mats, sig, stride,
+                               tiles, st, adj);
+    } else if (CAN_PP && L.pp_mass) {
+        hipLaunchKernelGGL((k_p2g<MODE, CAN_PP>), g, dim3(kP2GThreads), 0, s, A, P, L, mats, sig, stride, tiles, st,
+                           adj, skip_upto);
+    } else {
         hipLaunchKernelGGL((k_p2g<MODE, false>), g, dim3(kP2GThreads), 0, s, A, P, L, mats, sig, stride, tiles, st,
                            adj, skip_upto);
+    }
 }
 
 void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
@@ -2909,7 +3130,7 @@ void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const 
     // with sparse, blocks of <= kSparseMax particles go to the one-wave kernel (one chunk either way)
     const uint32_t skip = sparse ? (uint32_t)kSparseMax : 0u;
     if (!flush)
-        launch_p2g_mode<kP2GForward>(g, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, skip);
+        launch_p2g_mode<kP2GForward>(max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, skip);
     else if (L.pp_mass)
         hipLaunchKernelGGL((k_p2g<kP2GForward, true, true>), g, dim3(kP2GThreads), 0, s, A, P, L, mats, sig, stride,
                            tiles, st, AdjScatter{}, skip);
@@ -2924,17 +3145,15 @@ void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const 
 void launch_p2g_aflip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
                       float *tiles, float *tiles2, DevStatus *st, int64_t max_blocks, hipStream_t s) {
     if (max_blocks <= 0) return;
-    const dim3 g(persistent_grid(max_blocks, 1, 1 << 20));
-    launch_p2g_mode<kP2GMomentum>(g, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
-    launch_p2g_mode<kP2GStress>(g, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GMomentum>(max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GStress>(max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
 }
 
 void launch_p2g_flip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
                      float *tiles, float *tiles2, DevStatus *st, int64_t max_blocks, hipStream_t s) {
     if (max_blocks <= 0) return;
-    const dim3 g(persistent_grid(max_blocks, 1, 1 << 20));
-    launch_p2g_mode<kP2GFlipMomentum>(g, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
-    launch_p2g_mode<kP2GFlipStress>(g, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GFlipMomentum>(max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GFlipStress>(max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
 }
 
 void launch_grid_aflip(int mode, Partition P, Lattice L, const float *tiles, const float *tiles2, float *grid,
@@ -2948,8 +3167,7 @@ void launch_grid_aflip(int mode, Partition P, Lattice L, const float *tiles, con
 void launch_p2g_adjoint(State A, Partition P, Lattice L, AdjScatter adj, float *tiles, DevStatus *st,
                         int64_t max_blocks, hipStream_t s) {
     if (max_blocks <= 0) return;
-    hipLaunchKernelGGL(k_p2g<kP2GAdjoint>, dim3(persistent_grid(max_blocks, 1, 1 << 20)), dim3(kP2GThreads), 0, s, A,
-                       P, L, (const DevMaterial *)nullptr, (const float *)nullptr, (int64_t)0, tiles, st, adj, 0u);
+    launch_p2g_mode<kP2GAdjoint>(max_blocks, s, A, P, L, nullptr, nullptr, 0, tiles, st, adj, 0u);
 }
 
 void launch_grid(int mode, Partition P, Lattice L, const float *tiles, float *grid, float *gvmax,
