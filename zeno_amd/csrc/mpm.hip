@@ -2631,60 +2631,231 @@ __device__ __forceinline__ int64_t view_index(int layout, int64_t n, int tile_ch
     return ((i >> 5) * tile_ch + chn + c) * 32 + (i & 31);
 }
 
-// Particle j of the view becomes resident particle off + j, caller index off + j.
-__global__ void __launch_bounds__(kThreads) k_import(State dst, int64_t cap, zmpm_particles v, int64_t off,
-                                                     const DevMaterial *mats, int32_t nmat, DevStatus *st) {
+// Particle j of a view as the resident channels 0 .. kTileCh - 1 (all but kChPid): what the view does
+// not carry comes from its material.
+__device__ __forceinline__ int view_material(const zmpm_particles &v, int64_t j, int32_t nmat, bool &bad) {
+    const int32_t mid = v.material ? v.material[j] : v.default_material;
+    if (mid >= 0 && mid < nmat) return mid;
+    bad = true;
+    return 0;
+}
+
+__device__ __forceinline__ void view_channels(const zmpm_particles &v, int64_t j, const DevMaterial *mats,
+                                              int32_t nmat, bool &bad, float (&ch)[kTileCh]) {
     const int64_t n = v.n;
-    bool badmat = false;
-    for (int64_t j = blockIdx.x * (int64_t)kThreads + threadIdx.x; j < n; j += (int64_t)gridDim.x * kThreads) {
-        const int64_t i = off + j;
-        int32_t mid = v.material ? v.material[j] : v.default_material;
-        if (mid < 0 || mid >= nmat) {
-            badmat = true;
-            mid = 0;
-        }
-        const int model = mats[mid].model;
-        const bool fbased = model != ZMPM_MODEL_JFLUID;
+    const int mid = view_material(v, j, nmat, bad);
+    const bool fbased = mats[mid].model != ZMPM_MODEL_JFLUID;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            chan(dst.ch, i, c) = v.x[view_index(v.layout, n, v.tile_channels, v.x_chn, 3, c, j)];
-            chan(dst.ch, i, 3 + c) = v.v ? v.v[view_index(v.layout, n, v.tile_channels, v.v_chn, 3, c, j)] : 0.0f;
-        }
+    for (int c = 0; c < 3; ++c) {
+        ch[kChX + c] = v.x[view_index(v.layout, n, v.tile_channels, v.x_chn, 3, c, j)];
+        ch[kChV + c] = v.v ? v.v[view_index(v.layout, n, v.tile_channels, v.v_chn, 3, c, j)] : 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < 9; ++c) ch[kChC + c] = v.C ? v.C[view_index(v.layout, n, v.tile_channels, v.C_chn, 9, c, j)] : 0.0f;
+    if (fbased) {
 #pragma unroll
         for (int c = 0; c < 9; ++c)
-            chan(dst.ch, i, 6 + c) = v.C ? v.C[view_index(v.layout, n, v.tile_channels, v.C_chn, 9, c, j)] : 0.0f;
-        if (fbased) {
+            ch[kChF + c] = v.F ? v.F[view_index(v.layout, n, v.tile_channels, v.F_chn, 9, c, j)] : ((c % 4 == 0) ? 1.0f : 0.0f);
+    } else {
+        ch[kChF] = v.J ? v.J[view_index(v.layout, n, v.tile_channels, v.J_chn, 1, 0, j)] : 1.0f;
 #pragma unroll
-            for (int c = 0; c < 9; ++c)
-                chan(dst.ch, i, 15 + c) =
-                    v.F ? v.F[view_index(v.layout, n, v.tile_channels, v.F_chn, 9, c, j)] : ((c % 4 == 0) ? 1.0f : 0.0f);
-        } else {
-            chan(dst.ch, i, 15) = v.J ? v.J[view_index(v.layout, n, v.tile_channels, v.J_chn, 1, 0, j)] : 1.0f;
+        for (int c = 1; c < 9; ++c) ch[kChF + c] = 0.0f;
+    }
+    ch[kChMat] = __uint_as_float((uint32_t)mid | (fbased ? kMatF : 0u) |
+                                 (mats[mid].plasticity != ZMPM_PLASTIC_NONE ? kMatPlastic : 0u));
+    ch[kChBeta] = v.beta ? v.beta[view_index(v.layout, n, v.tile_channels, v.beta_chn, 1, 0, j)] : mats[mid].flip_beta;
+    ch[kChLogJp] = v.logJp ? v.logJp[view_index(v.layout, n, v.tile_channels, v.logJp_chn, 1, 0, j)] : kLogJpInit;
+    const bool pp = v.mu && v.lam;
+    ch[kChMu] = pp ? v.mu[view_index(v.layout, n, v.tile_channels, v.mu_chn, 1, 0, j)] : mats[mid].mu;
+    ch[kChLam] = pp ? v.lam[view_index(v.layout, n, v.tile_channels, v.lam_chn, 1, 0, j)] : mats[mid].lam;
+    // the fiber "a", (0, 1, 0) when none is given (Generation.cpp:982)
 #pragma unroll
-            for (int c = 1; c < 9; ++c) chan(dst.ch, i, 15 + c) = 0.0f;
-        }
-        set_u(dst.ch, (uint32_t)i, kChMat,
-              (uint32_t)mid | (fbased ? kMatF : 0u) | (mats[mid].plasticity != ZMPM_PLASTIC_NONE ? kMatPlastic : 0u));
-        set_u(dst.ch, (uint32_t)i, kChPid, (uint32_t)i);
-        chan(dst.ch, i, kChBeta) =
-            v.beta ? v.beta[view_index(v.layout, n, v.tile_channels, v.beta_chn, 1, 0, j)] : mats[mid].flip_beta;
-        chan(dst.ch, i, kChLogJp) =
-            v.logJp ? v.logJp[view_index(v.layout, n, v.tile_channels, v.logJp_chn, 1, 0, j)] : kLogJpInit;
-        const bool pp = v.mu && v.lam;
-        chan(dst.ch, i, kChMu) = pp ? v.mu[view_index(v.layout, n, v.tile_channels, v.mu_chn, 1, 0, j)] : mats[mid].mu;
-        chan(dst.ch, i, kChLam) =
-            pp ? v.lam[view_index(v.layout, n, v.tile_channels, v.lam_chn, 1, 0, j)] : mats[mid].lam;
-        // the fiber "a", (0, 1, 0) when none is given (Generation.cpp:982)
+    for (int c = 0; c < 3; ++c)
+        ch[kChFiber + c] = v.a ? v.a[view_index(v.layout, n, v.tile_channels, v.a_chn, 3, c, j)] : (c == 1 ? 1.0f : 0.0f);
+    // per-particle mass and volume (Transfer.cu:857-858), else the material's
+    const bool pm = v.m && v.vol;
+    ch[kChMass] = pm ? v.m[view_index(v.layout, n, v.tile_channels, v.m_chn, 1, 0, j)] : mats[mid].mass;
+    ch[kChVol] = pm ? v.vol[view_index(v.layout, n, v.tile_channels, v.vol_chn, 1, 0, j)] : mats[mid].vol;
+}
+
+// Particle j of the view becomes resident particle off + j, caller index off + j.
+__global__ void __launch_bounds__(kThreads) k_import(State dst, zmpm_particles v, int64_t off,
+                                                     const DevMaterial *mats, int32_t nmat, DevStatus *st) {
+    bool badmat = false;
+    for (int64_t j = blockIdx.x * (int64_t)kThreads + threadIdx.x; j < v.n; j += (int64_t)gridDim.x * kThreads) {
+        float ch[kTileCh];
+        view_channels(v, j, mats, nmat, badmat, ch);
+        ch[kChPid] = __uint_as_float((uint32_t)(off + j));
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-            chan(dst.ch, i, kChFiber + c) =
-                v.a ? v.a[view_index(v.layout, n, v.tile_channels, v.a_chn, 3, c, j)] : (c == 1 ? 1.0f : 0.0f);
-        // per-particle mass and volume (Transfer.cu:857-858), else the material's
-        const bool pm = v.m && v.vol;
-        chan(dst.ch, i, kChMass) = pm ? v.m[view_index(v.layout, n, v.tile_channels, v.m_chn, 1, 0, j)] : mats[mid].mass;
-        chan(dst.ch, i, kChVol) = pm ? v.vol[view_index(v.layout, n, v.tile_channels, v.vol_chn, 1, 0, j)] : mats[mid].vol;
+        for (int c = 0; c < kTileCh; ++c) chan(dst.ch, (uint32_t)(off + j), c) = ch[c];
     }
     if (badmat) atomicOr(&st->bad_material, 1u);
+}
+
+// ------------------------------------------------------------------ reordering through records
+// A permutation of particles whose channels lie in planes or tiles reads (or writes) four bytes of a
+// cache line per particle and channel when the order is far from the memory's.  Such a one goes
+// through records instead: kRec floats of a particle in one 128-byte line.  One pass turns channels
+// into records, coalesced on both sides through LDS; the permuted side moves whole lines.  That
+// doubles the bytes (4.9 million particles of 256 scenes: export 1,936 -> 238 + 261 us, at 5 TB/s; a
+// shuffled 613,057: import and sort by 35 + 27 us for 48 + 240), so an order that is local (runs of a wave's 64 entries in few lines) keeps the
+// direct kernels.  k_order_sample decides on the device, without a synchronisation: both kinds are
+// launched and one returns at once.
+constexpr int kRec = 32;
+constexpr int kRecPitch = 36;  // floats of a record's row in LDS: 16-byte rows on distinct banks
+constexpr int kRecWaves = kThreads / 64;
+
+// The channels of a record other than 0 .. kChMat, which keep their places.
+constexpr int kRecBeta = 25, kRecLogJp = 26, kRecMu = 27, kRecLam = 28, kRecMass = 29, kRecVol = 30;
+
+// Lane l's v to record idx (of its own; kNoRec: none) / from it.  s: the wave's 64 LDS rows.
+constexpr uint32_t kNoRec = 0xffffffffu;
+__device__ __forceinline__ void rec_put(float *s, const float (&v)[kRec], float *rec, uint32_t idx) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < kRec; q += 4)
+        *reinterpret_cast<float4 *>(s + lane * kRecPitch + q) = make_float4(v[q], v[q + 1], v[q + 2], v[q + 3]);
+    wave_lds_order();
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {  // eight lanes write one record
+        const int r = it * 8 + (lane >> 3);
+        const uint32_t at = (uint32_t)__shfl((int)idx, r, 64);
+        const float4 x = *reinterpret_cast<const float4 *>(s + r * kRecPitch + 4 * (lane & 7));
+        if (at != kNoRec) *reinterpret_cast<float4 *>(rec + (size_t)at * kRec + 4 * (lane & 7)) = x;
+    }
+    wave_lds_order();
+}
+
+__device__ __forceinline__ void rec_get(float *s, float (&v)[kRec], const float *rec, uint32_t idx) {
+    const int lane = threadIdx.x & 63;
+    float4 x[8];
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+        const uint32_t at = (uint32_t)__shfl((int)idx, it * 8 + (lane >> 3), 64);
+        x[it] = at != kNoRec ? *reinterpret_cast<const float4 *>(rec + (size_t)at * kRec + 4 * (lane & 7))
+                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int it = 0; it < 8; ++it)
+        *reinterpret_cast<float4 *>(s + (it * 8 + (lane >> 3)) * kRecPitch + 4 * (lane & 7)) = x[it];
+    wave_lds_order();
+#pragma unroll
+    for (int q = 0; q < kRec; q += 4) {
+        const float4 y = *reinterpret_cast<const float4 *>(s + lane * kRecPitch + q);
+        v[q] = y.x;
+        v[q + 1] = y.y;
+        v[q + 2] = y.z;
+        v[q + 3] = y.w;
+    }
+    wave_lds_order();
+}
+
+// *staged = the order (perm, or the caller indices of the resident particles) is far from the
+// memory's: 64 runs of 64 entries, evenly over the n >= 64, hold more than kLocalLines different
+// lines of 32 entries each on average (neighbours compared, so a line met again counts again).
+// 2,000,000 particles shuffled within windows of 1, 64, 256, 4,096 and all entries hold 7, 10, 25, 47
+// and 64 lines: an export takes 184, 218, 369, 638 and 972 us directly, 205 through records; an
+// import with its sort 319, 347, 417, 522 and 1,057, against 385.  At 600,000 the export: 63, 82, 116,
+// 159 and 203, against 71.
+constexpr uint32_t kLocalLines = 12;
+__global__ void __launch_bounds__(1024) k_order_sample(const uint32_t *perm, const float *ch, int64_t n,
+                                                       uint32_t *staged) {
+    __shared__ uint32_t s_lines[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t lines = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int64_t k = (n - 64) * (4 * w + q) / 63 + lane;
+        const uint32_t line = (perm ? perm[k] : chan_u(ch, (uint32_t)k, kChPid)) >> 5;
+        const uint32_t prev = (uint32_t)__shfl_up((int)line, 1, 64);
+        lines += (uint32_t)__popcll(__ballot(lane == 0 || line != prev));
+    }
+    if (lane == 0) s_lines[w] = lines;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t total = 0;
+        for (int q = 0; q < 16; ++q) total += s_lines[q];
+        *staged = total > 64u * kLocalLines ? 1u : 0u;
+    }
+}
+
+// Keys of the view's particles, as k_bin_keys makes them from the resident ones.
+__global__ void __launch_bounds__(kThreads) k_view_keys(zmpm_particles v, int64_t off, const DevMaterial *mats,
+                                                        int32_t nmat, Lattice L, uint32_t *keys, DevStatus *st) {
+    bool bad = false, badmat = false;
+    for (int64_t j = blockIdx.x * (int64_t)kThreads + threadIdx.x; j < v.n; j += (int64_t)gridDim.x * kThreads) {
+        const int mid = view_material(v, j, nmat, badmat);
+        float xp[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) xp[c] = v.x[view_index(v.layout, v.n, v.tile_channels, v.x_chn, 3, c, j)];
+        keys[off + j] = position_key(xp, scene_params(L, (uint32_t)mats[mid].scene), L.origin, L.key_shift, bad);
+    }
+    if (bad) atomicOr(&st->domain_error, 1u);
+    if (badmat) atomicOr(&st->bad_material, 1u);
+}
+
+// View -> records at the caller index (the view carries no fiber).
+__global__ void __launch_bounds__(kThreads) k_view_to_rec(zmpm_particles v, int64_t off, const DevMaterial *mats,
+                                                          int32_t nmat, float *rec, const uint32_t *staged) {
+    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    if (staged && *staged == 0u) return;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    bool bad = false;
+    for (int64_t j0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; j0 < v.n; j0 += (int64_t)gridDim.x * kThreads) {
+        const int64_t j = j0 + lane;
+        float ch[kTileCh], r[kRec];
+        view_channels(v, min(j, v.n - 1), mats, nmat, bad, ch);
+#pragma unroll
+        for (int c = 0; c <= kChMat; ++c) r[c] = ch[c];
+        r[kRecBeta] = ch[kChBeta];
+        r[kRecLogJp] = ch[kChLogJp];
+        r[kRecMu] = ch[kChMu];
+        r[kRecLam] = ch[kChLam];
+        r[kRecMass] = ch[kChMass];
+        r[kRecVol] = ch[kChVol];
+        r[kRec - 1] = 0.0f;
+        rec_put(s_rec[w], r, rec, j < v.n ? (uint32_t)(off + j) : kNoRec);
+    }
+}
+
+// Caller particle perm[k] becomes resident particle k: from the records, or (DIRECT) from the view of
+// all particles.
+template <bool DIRECT>
+__global__ void __launch_bounds__(kThreads) k_import_sorted(State dst, zmpm_particles v, const float *rec,
+                                                            const uint32_t *perm, int64_t n, const DevMaterial *mats,
+                                                            int32_t nmat, const uint32_t *staged) {
+    __shared__ float s_rec[DIRECT ? 1 : kRecWaves][64 * kRecPitch];
+    if (staged && (*staged != 0u) == DIRECT) return;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    bool bad = false;
+    for (int64_t k0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; k0 < n; k0 += (int64_t)gridDim.x * kThreads) {
+        const int64_t k = k0 + lane;
+        const uint32_t i = perm[min(k, n - 1)];
+        float ch[kTileCh];
+        if (DIRECT) {
+            view_channels(v, i, mats, nmat, bad, ch);
+        } else {
+            float r[kRec];
+            rec_get(s_rec[w], r, rec, i);
+#pragma unroll
+            for (int c = 0; c <= kChMat; ++c) ch[c] = r[c];
+            ch[kChBeta] = r[kRecBeta];
+            ch[kChLogJp] = r[kRecLogJp];
+            ch[kChMu] = r[kRecMu];
+            ch[kChLam] = r[kRecLam];
+            ch[kChMass] = r[kRecMass];
+            ch[kChVol] = r[kRecVol];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) ch[kChFiber + c] = c == 1 ? 1.0f : 0.0f;
+        }
+        ch[kChPid] = __uint_as_float(i);
+        if (k < n) {
+#pragma unroll
+            for (int c = 0; c < kTileCh; ++c) chan(dst.ch, (uint32_t)k, c) = ch[c];
+        }
+    }
 }
 
 // ------------------------------------------------------------------ Morton order
@@ -2727,9 +2898,13 @@ __global__ void __launch_bounds__(kThreads) k_morton_codes(int32_t layout, int32
     }
 }
 
-// Every channel of particle order[k] of src becomes particle k of dst (Structures.hpp:438-443).
+// Every channel of particle order[k] of src becomes particle k of dst (Structures.hpp:438-443):
+// directly, or through records (nch <= kRec).  1,048,583 particles of 28 channels in no order: 500 us
+// directly, 47 + 51 us through records.
 __global__ void __launch_bounds__(kThreads) k_permute_channels(int32_t layout, int32_t nch, int64_t n,
-                                                               const float *src, float *dst, const uint32_t *order) {
+                                                               const float *src, float *dst, const uint32_t *order,
+                                                               const uint32_t *staged) {
+    if (staged && *staged != 0u) return;
     for (int64_t k = blockIdx.x * (int64_t)kThreads + threadIdx.x; k < n; k += (int64_t)gridDim.x * kThreads) {
         const int64_t i = order[k];
         for (int c = 0; c < nch; ++c)
@@ -2737,11 +2912,44 @@ __global__ void __launch_bounds__(kThreads) k_permute_channels(int32_t layout, i
     }
 }
 
+__global__ void __launch_bounds__(kThreads) k_channels_to_rec(int32_t layout, int32_t nch, int64_t n, const float *src,
+                                                              float *rec, const uint32_t *staged) {
+    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    if (*staged == 0u) return;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int64_t k0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; k0 < n; k0 += (int64_t)gridDim.x * kThreads) {
+        const int64_t k = k0 + lane;
+        float r[kRec];
+#pragma unroll
+        for (int c = 0; c < kRec; ++c) r[c] = c < nch && k < n ? src[buf_index(layout, n, nch, c, k)] : 0.0f;
+        rec_put(s_rec[w], r, rec, k < n ? (uint32_t)k : kNoRec);
+    }
+}
+
+__global__ void __launch_bounds__(kThreads) k_rec_to_channels(int32_t layout, int32_t nch, int64_t n, const float *rec,
+                                                              float *dst, const uint32_t *order,
+                                                              const uint32_t *staged) {
+    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    if (*staged == 0u) return;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int64_t k0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; k0 < n; k0 += (int64_t)gridDim.x * kThreads) {
+        const int64_t k = k0 + lane;
+        float r[kRec];
+        rec_get(s_rec[w], r, rec, k < n ? order[k] : kNoRec);
+#pragma unroll
+        for (int c = 0; c < kRec; ++c)
+            if (c < nch && k < n) dst[buf_index(layout, n, nch, c, k)] = r[c];
+    }
+}
+
 // aux: the kAux* channels the resident state keeps; the others are exported
 // as their initial values (the material's flip_beta, logJp -0.04).
 // Resident particles of caller index off .. off + v.n - 1 go to the view's entries 0 .. v.n - 1.
 __global__ void __launch_bounds__(kThreads) k_export(State src, int64_t n_res, zmpm_particles v, int64_t off,
-                                                     const DevMaterial *mats, int aux) {
+                                                     const DevMaterial *mats, int aux, const uint32_t *staged) {
+    if (staged && *staged != 0u) return;
     const int64_t n = v.n;
     for (int64_t k = blockIdx.x * (int64_t)kThreads + threadIdx.x; k < n_res; k += (int64_t)gridDim.x * kThreads) {
         const int64_t i = (int64_t)chan_u(src.ch, (uint32_t)k, kChPid) - off;
@@ -2790,6 +2998,81 @@ __global__ void __launch_bounds__(kThreads) k_export(State src, int64_t n_res, z
             }
         } else if (v.J) {
             v.J[view_index(v.layout, n, v.tile_channels, v.J_chn, 1, 0, i)] = chan(src.ch, k, 15);
+        }
+    }
+}
+
+// The same through records: resident particles -> records at their caller index -> the views.
+// want: the kAux* channels that a view asks for.
+__global__ void __launch_bounds__(kThreads) k_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux,
+                                                            int want, float *rec, const uint32_t *staged) {
+    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    if (*staged == 0u) return;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int64_t k0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; k0 < n; k0 += (int64_t)gridDim.x * kThreads) {
+        const uint32_t k = (uint32_t)min(k0 + lane, n - 1);
+        const uint32_t mw = chan_u(src.ch, k, kChMat);
+        float r[kRec];
+#pragma unroll
+        for (int c = 0; c <= kChF; ++c) r[c] = chan(src.ch, k, c);
+#pragma unroll
+        for (int c = kChF + 1; c < kChMat; ++c) r[c] = (mw & kMatF) ? chan(src.ch, k, c) : 0.0f;
+        r[kChMat] = __uint_as_float(mw);
+#pragma unroll
+        for (int c = kChMat + 1; c < kRec; ++c) r[c] = 0.0f;
+        if (want) {
+            const DevMaterial &mt = mats[mw & kMatIndexMask];
+            if (want & kAuxBeta) r[kRecBeta] = (aux & kAuxBeta) ? chan(src.ch, k, kChBeta) : mt.flip_beta;
+            if (want & kAuxLogJp) r[kRecLogJp] = (aux & kAuxLogJp) ? chan(src.ch, k, kChLogJp) : kLogJpInit;
+            if (want & kAuxLame) {
+                r[kRecMu] = (aux & kAuxLame) ? chan(src.ch, k, kChMu) : mt.mu;
+                r[kRecLam] = (aux & kAuxLame) ? chan(src.ch, k, kChLam) : mt.lam;
+            }
+            if (want & kAuxMass) {
+                r[kRecMass] = (aux & kAuxMass) ? chan(src.ch, k, kChMass) : mt.mass;
+                r[kRecVol] = (aux & kAuxMass) ? chan(src.ch, k, kChVol) : mt.vol;
+            }
+        }
+        rec_put(s_rec[w], r, rec, k0 + lane < n ? chan_u(src.ch, k, kChPid) : kNoRec);
+    }
+}
+
+// Records off .. off + v.n - 1 to the view (which asks for no fiber).
+__global__ void __launch_bounds__(kThreads) k_rec_to_view(const float *rec, zmpm_particles v, int64_t off,
+                                                          const uint32_t *staged) {
+    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    if (*staged == 0u) return;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t n = v.n;
+    for (int64_t i0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; i0 < n; i0 += (int64_t)gridDim.x * kThreads) {
+        const int64_t i = i0 + lane;
+        float r[kRec];
+        rec_get(s_rec[w], r, rec, i < n ? (uint32_t)(off + i) : kNoRec);
+        if (i >= n) continue;
+        if (v.beta) v.beta[view_index(v.layout, n, v.tile_channels, v.beta_chn, 1, 0, i)] = r[kRecBeta];
+        if (v.logJp) v.logJp[view_index(v.layout, n, v.tile_channels, v.logJp_chn, 1, 0, i)] = r[kRecLogJp];
+        if (v.mu) v.mu[view_index(v.layout, n, v.tile_channels, v.mu_chn, 1, 0, i)] = r[kRecMu];
+        if (v.lam) v.lam[view_index(v.layout, n, v.tile_channels, v.lam_chn, 1, 0, i)] = r[kRecLam];
+        if (v.m) v.m[view_index(v.layout, n, v.tile_channels, v.m_chn, 1, 0, i)] = r[kRecMass];
+        if (v.vol) v.vol[view_index(v.layout, n, v.tile_channels, v.vol_chn, 1, 0, i)] = r[kRecVol];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            v.x[view_index(v.layout, n, v.tile_channels, v.x_chn, 3, c, i)] = r[c];
+            if (v.v) v.v[view_index(v.layout, n, v.tile_channels, v.v_chn, 3, c, i)] = r[kChV + c];
+        }
+        if (v.C) {
+#pragma unroll
+            for (int c = 0; c < 9; ++c) v.C[view_index(v.layout, n, v.tile_channels, v.C_chn, 9, c, i)] = r[kChC + c];
+        }
+        if (__float_as_uint(r[kChMat]) & kMatF) {
+            if (v.F) {
+#pragma unroll
+                for (int c = 0; c < 9; ++c) v.F[view_index(v.layout, n, v.tile_channels, v.F_chn, 9, c, i)] = r[kChF + c];
+            }
+        } else if (v.J) {
+            v.J[view_index(v.layout, n, v.tile_channels, v.J_chn, 1, 0, i)] = r[kChF];
         }
     }
 }
@@ -3247,9 +3530,18 @@ void launch_morton_codes(int32_t layout, int32_t nch, int64_t n, const float *sr
 }
 
 void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float *src, float *dst,
-                             const uint32_t *order, hipStream_t s) {
+                             const uint32_t *order, float *rec, uint32_t *staged, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_permute_channels, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, layout, nch, n, src, dst, order);
+    const bool staging = rec && nch <= kRec && layout != ZMPM_LAYOUT_AOS && n >= kStageMin;
+    if (staging) {
+        launch_order_sample(order, State{}, n, staged, s);
+        hipLaunchKernelGGL(k_channels_to_rec, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, layout, nch, n, src, rec,
+                           (const uint32_t *)staged);
+        hipLaunchKernelGGL(k_rec_to_channels, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, layout, nch, n,
+                           (const float *)rec, dst, order, (const uint32_t *)staged);
+    }
+    hipLaunchKernelGGL(k_permute_channels, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, layout, nch, n, src, dst,
+                       order, staging ? (const uint32_t *)staged : nullptr);
 }
 
 void launch_lattice_scan(Lattice L, Partition Pn, Binning B, const uint32_t *prev_used, int64_t n, DevStatus *st,
@@ -3296,11 +3588,40 @@ void launch_g2p_update(bool scatter, State A, State Bst, Partition P, Partition 
         hipLaunchKernelGGL((k_g2p_update<false, kThreads>), dim3(g), dim3(kThreads), 0, s, u);
 }
 
-void launch_import(State dst, int64_t cap, const void *view, int64_t off, const DevMaterial *mats, int32_t nmat,
-                   DevStatus *st, hipStream_t s) {
+void launch_import(State dst, const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, DevStatus *st,
+                   hipStream_t s) {
     const zmpm_particles v = *(const zmpm_particles *)view;
     if (v.n <= 0) return;
-    hipLaunchKernelGGL(k_import, dim3(grid_for(v.n, 8192)), dim3(kThreads), 0, s, dst, cap, v, off, mats, nmat, st);
+    hipLaunchKernelGGL(k_import, dim3(grid_for(v.n, 8192)), dim3(kThreads), 0, s, dst, v, off, mats, nmat, st);
+}
+
+void launch_order_sample(const uint32_t *perm, State A, int64_t n, uint32_t *staged, hipStream_t s) {
+    hipLaunchKernelGGL(k_order_sample, dim3(1), dim3(1024), 0, s, perm, (const float *)A.ch, n, staged);
+}
+
+void launch_view_keys(const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, Lattice L, uint32_t *keys,
+                      DevStatus *st, hipStream_t s) {
+    const zmpm_particles v = *(const zmpm_particles *)view;
+    if (v.n <= 0) return;
+    hipLaunchKernelGGL(k_view_keys, dim3(grid_for(v.n, 8192)), dim3(kThreads), 0, s, v, off, mats, nmat, L, keys, st);
+}
+
+void launch_view_to_rec(const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, float *rec,
+                        const uint32_t *staged, hipStream_t s) {
+    const zmpm_particles v = *(const zmpm_particles *)view;
+    if (v.n <= 0) return;
+    hipLaunchKernelGGL(k_view_to_rec, dim3(grid_for(v.n, 4096)), dim3(kThreads), 0, s, v, off, mats, nmat, rec, staged);
+}
+
+void launch_import_sorted(State dst, const void *view, const float *rec, const uint32_t *perm, int64_t n,
+                          const DevMaterial *mats, int32_t nmat, const uint32_t *staged, hipStream_t s) {
+    if (n <= 0) return;
+    if (rec)
+        hipLaunchKernelGGL(k_import_sorted<false>, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, dst,
+                           zmpm_particles{}, rec, perm, n, mats, nmat, staged);
+    if (view)
+        hipLaunchKernelGGL(k_import_sorted<true>, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, dst,
+                           *(const zmpm_particles *)view, (const float *)nullptr, perm, n, mats, nmat, staged);
 }
 
 void launch_colliders(Partition P, Lattice L, float *grid, float *gvmax, int64_t max_blocks, bool vmax,
@@ -3355,10 +3676,23 @@ void launch_particle_volume(State A, int64_t n, Partition P, Lattice L, const De
 }
 
 void launch_export(State src, int64_t n_res, const void *view, int64_t off, const DevMaterial *mats, int aux,
-                   hipStream_t s) {
+                   const uint32_t *staged, hipStream_t s) {
     const zmpm_particles v = *(const zmpm_particles *)view;
     if (v.n <= 0 || n_res <= 0) return;
-    hipLaunchKernelGGL(k_export, dim3(grid_for(n_res, 8192)), dim3(kThreads), 0, s, src, n_res, v, off, mats, aux);
+    hipLaunchKernelGGL(k_export, dim3(grid_for(n_res, 8192)), dim3(kThreads), 0, s, src, n_res, v, off, mats, aux,
+                       staged);
+}
+
+void launch_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux, int want, float *rec,
+                          const uint32_t *staged, hipStream_t s) {
+    hipLaunchKernelGGL(k_export_to_rec, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, src, n, mats, aux, want, rec,
+                       staged);
+}
+
+void launch_rec_to_view(const float *rec, const void *view, int64_t off, const uint32_t *staged, hipStream_t s) {
+    const zmpm_particles v = *(const zmpm_particles *)view;
+    if (v.n <= 0) return;
+    hipLaunchKernelGGL(k_rec_to_view, dim3(grid_for(v.n, 4096)), dim3(kThreads), 0, s, rec, v, off, staged);
 }
 
 }  // namespace zmpm

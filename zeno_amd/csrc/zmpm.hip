@@ -104,6 +104,9 @@ struct zmpm_ctx {
     int grid_part = 0;  // the partition the grid values belong to
 
     uint32_t *keys = nullptr, *skeys = nullptr, *perm = nullptr;
+    uint32_t *staged = nullptr;  // k_order_sample's word
+    // between calls st[cur ^ 1] holds nothing: the records of an export or a reordering lie there
+    float *records() const { return st[cur ^ 1].ch; }
     void *sort_scratch = nullptr;
     Binning bin{};
     float *tiles = nullptr, *grid = nullptr;
@@ -235,27 +238,53 @@ void check_status(zmpm_ctx *c) {
         throw ZmpmError(ZMPM_ERR_STATE, "internal binning inconsistency (bin mismatch or look-back stall)");
 }
 
+// Stable sort of the keys by block (the key bits above the 6 cell bits) into skeys, perm.
+void sort_by_block(zmpm_ctx *c) {
+    radix_sort_pairs(c->keys, nullptr, c->n, c->L.key_shift, c->key_bits, c->skeys, c->perm, nullptr,
+                     c->sort_scratch, c->stream);
+}
+
+// One view of all particles, or several through records: the particles into block order in
+// st[cur ^ 1], which then is the resident state.
+void import_sorted(zmpm_ctx *c, const zmpm_particles *views, int32_t nviews, bool records) {
+    hipStream_t s = c->stream;
+    int64_t off = 0;
+    for (int k = 0; k < nviews; off += views[k++].n)
+        launch_view_keys(&views[k], off, c->mats, c->nmat, c->L, c->keys, c->status, s);
+    sort_by_block(c);
+    float *rec = records ? c->st[c->cur].ch : nullptr;
+    uint32_t *staged = records && nviews == 1 ? c->staged : nullptr;
+    if (staged) launch_order_sample(c->perm, State{}, c->n, staged, s);
+    off = 0;
+    for (int k = 0; rec && k < nviews; off += views[k++].n)
+        launch_view_to_rec(&views[k], off, c->mats, c->nmat, rec, staged, s);
+    launch_import_sorted(c->st[c->cur ^ 1], nviews == 1 ? views : nullptr, rec, c->perm, c->n, c->mats, c->nmat,
+                         staged, s);
+    c->cur ^= 1;
+    c->loaded_sorted = false;
+}
+
 // Bin the resident particles: keys -> stable sort -> permute the state into
 // sorted order -> particle blocks and grid blocks (B + {0,1}^3).
 // part_shift: the parts (of 2^part_shift particles) to cut the blocks into (0: what the context's
-// chain wants).
-void full_partition(zmpm_ctx *c, uint32_t part_shift = 0) {
+// chain wants).  sorted: import_sorted has done the keys, the sort and the permutation.
+void full_partition(zmpm_ctx *c, uint32_t part_shift = 0, bool sorted = false) {
     hipStream_t s = c->stream;
     c->L.part_shift = part_shift ? part_shift : c->wanted_part_shift();
     c->psize[c->pcur] = c->L.part_shift;
     State A = c->st[c->cur], B = c->st[c->cur ^ 1];
     // a saved state is already in stable block order: the sort would be the identity
     // (a state that is not is reported as a binning inconsistency at the next sync)
-    launch_bin_keys(A.ch, -1, c->n, c->mats, c->L, c->keys, c->status, s, c->loaded_sorted);
+    if (!sorted) launch_bin_keys(A.ch, -1, c->n, c->mats, c->L, c->keys, c->status, s, c->loaded_sorted);
     if (c->loaded_sorted) {
         launch_partition_from_keys(c->keys, c->n, c->L, c->part[c->pcur], c->bin, A, c->mats, c->status, s);
         c->loaded_sorted = false;
     } else {
-        // stable sort by block (key bits above the 6 cell bits)
-        radix_sort_pairs(c->keys, nullptr, c->n, c->L.key_shift, c->key_bits, c->skeys, c->perm, nullptr,
-                         c->sort_scratch, s);
-        launch_gather_state(A, c->cap, B, c->cap, c->perm, c->n, s);
-        c->cur ^= 1;
+        if (!sorted) {
+            sort_by_block(c);
+            launch_gather_state(A, c->cap, B, c->cap, c->perm, c->n, s);
+            c->cur ^= 1;
+        }
         launch_partition_from_keys(c->skeys, c->n, c->L, c->part[c->pcur], c->bin, c->st[c->cur], c->mats,
                                    c->status, s);
     }
@@ -393,6 +422,7 @@ zmpm_ctx *create_context(const zmpm_scene *scenes, int32_t nscenes, int64_t capa
         c->keys = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->skeys = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->perm = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
+        c->staged = (uint32_t *)c->alloc(sizeof(uint32_t));
         c->sort_scratch = c->alloc(radix_scratch_bytes(cap));
         c->tiles = (float *)c->alloc(sizeof(float) * 4 * kTileNodes * parts_cap);
         c->tiles_blocks = parts_cap;
@@ -612,13 +642,19 @@ void import_views(zmpm_ctx *ctx, const zmpm_particles *views, int32_t nviews) {
     ctx->pp_mass = mass;
     ctx->sync_pp_flag();
     fill_u32((uint32_t *)ctx->status, 0u, sizeof(DevStatus) / 4, ctx->stream);
-    int64_t off = 0;
-    for (int k = 0; k < nviews; ++k) {
-        launch_import(ctx->st[ctx->cur], ctx->cap, &views[k], off, ctx->mats, ctx->nmat, ctx->status, ctx->stream);
-        off += views[k].n;
+    bool fibers = false;
+    for (int k = 0; k < nviews; ++k) fibers = fibers || views[k].a;
+    const bool records = total >= kStageMin && !fibers;
+    const bool sorted = nviews == 1 || records;
+    if (sorted) {
+        import_sorted(ctx, views, nviews, records);
+    } else {
+        int64_t off = 0;
+        for (int k = 0; k < nviews; off += views[k++].n)
+            launch_import(ctx->st[ctx->cur], &views[k], off, ctx->mats, ctx->nmat, ctx->status, ctx->stream);
     }
     HIP_CHECK(hipGetLastError());
-    full_partition(ctx);
+    full_partition(ctx, 0, sorted);
     check_status(ctx);
 }
 
@@ -627,10 +663,20 @@ void export_views(zmpm_ctx *ctx, const zmpm_particles *views, int32_t nviews) {
     if (check_views(views, nviews) != ctx->n)
         throw ZmpmError(ZMPM_ERR_ARG, "export views must cover exactly the imported particles");
     ctx->set_device();
+    int want = 0;
+    for (int k = 0; k < nviews; ++k)
+        want |= (views[k].beta ? kAuxBeta : 0) | (views[k].logJp ? kAuxLogJp : 0) | (views[k].mu ? kAuxLame : 0) |
+                (views[k].a ? kAuxFiber : 0) | (views[k].m ? kAuxMass : 0);
+    uint32_t *staged = ctx->n >= kStageMin && !(want & kAuxFiber) ? ctx->staged : nullptr;
+    if (staged) {
+        launch_order_sample(nullptr, ctx->st[ctx->cur], ctx->n, staged, ctx->stream);
+        launch_export_to_rec(ctx->st[ctx->cur], ctx->n, ctx->mats, ctx->aux(), want, ctx->records(), staged,
+                             ctx->stream);
+    }
     int64_t off = 0;
-    for (int k = 0; k < nviews; ++k) {
-        launch_export(ctx->st[ctx->cur], ctx->n, &views[k], off, ctx->mats, ctx->aux(), ctx->stream);
-        off += views[k].n;
+    for (int k = 0; k < nviews; off += views[k++].n) {
+        if (staged) launch_rec_to_view(ctx->records(), &views[k], off, staged, ctx->stream);
+        launch_export(ctx->st[ctx->cur], ctx->n, &views[k], off, ctx->mats, ctx->aux(), staged, ctx->stream);
     }
     HIP_CHECK(hipGetLastError());
     check_status(ctx);
@@ -1638,7 +1684,16 @@ int32_t zmpm_order_by_morton_code(zmpm_ctx *ctx, int32_t layout, int32_t nch, in
         radix_sort_pairs(ctx->keys, nullptr, n, 0, 30, codes ? codes : ctx->skeys,
                          reinterpret_cast<uint32_t *>(ordered_to_original),
                          reinterpret_cast<uint32_t *>(original_to_ordered), ctx->sort_scratch, s);
-        launch_permute_channels(layout, nch, n, src, dst, reinterpret_cast<const uint32_t *>(ordered_to_original), s);
+        // a captured launch may run when st[cur ^ 1] holds the state: it permutes directly
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        bool free_buffer = true;
+        if (hipStreamIsCapturing(s, &capture) != hipSuccess) {
+            (void)hipGetLastError();
+            free_buffer = false;
+        }
+        free_buffer = free_buffer && capture == hipStreamCaptureStatusNone;
+        launch_permute_channels(layout, nch, n, src, dst, reinterpret_cast<const uint32_t *>(ordered_to_original),
+                                free_buffer ? ctx->records() : nullptr, ctx->staged, s);
         HIP_CHECK(hipGetLastError());
     });
 }

@@ -309,12 +309,33 @@ void launch_grid_aflip(int mode, Partition P, Lattice L, const float *tiles, con
                        int32_t nclear = 0);
 // view: a const zmpm_particles* (device pointers inside); its particle i becomes resident
 // particle off + i with caller index off + i (one object of a list of particle objects)
-void launch_import(State dst, int64_t cap, const void *view, int64_t off, const DevMaterial *mats, int32_t nmat,
-                   DevStatus *st, hipStream_t s);
-// aux: the kAux* channels the resident state keeps (the others are exported as their initial values);
-// the resident particles of caller index off .. off + view->n - 1 go to the view's entries 0 .. n - 1
-void launch_export(State src, int64_t n_res, const void *view, int64_t off, const DevMaterial *mats, int aux,
+void launch_import(State dst, const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, DevStatus *st,
                    hipStream_t s);
+// Import in block order: the keys of a view's particles, then (after the sort) resident particle k =
+// caller particle perm[k], from the view of all particles (view), from records of 32 floats per caller
+// particle (rec, made by launch_view_to_rec), or, both given, from what *staged says.
+// Records are used from kStageMin particles on (65,536 shuffled: export 38 us through records, 45
+// directly, import 160 and 157; below, the launches cost more than they give) and hold every
+// attribute but the fiber.
+constexpr int64_t kStageMin = 65536;
+void launch_view_keys(const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, Lattice L, uint32_t *keys,
+                      DevStatus *st, hipStream_t s);
+void launch_view_to_rec(const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, float *rec,
+                        const uint32_t *staged, hipStream_t s);
+void launch_import_sorted(State dst, const void *view, const float *rec, const uint32_t *perm, int64_t n,
+                          const DevMaterial *mats, int32_t nmat, const uint32_t *staged, hipStream_t s);
+// *staged = whether perm (null: the resident particles' caller indices) is so far from memory order
+// that moving the particles through records is the faster way (n >= 64)
+void launch_order_sample(const uint32_t *perm, State A, int64_t n, uint32_t *staged, hipStream_t s);
+// aux: the kAux* channels the resident state keeps (the others are exported as their initial values);
+// the resident particles of caller index off .. off + view->n - 1 go to the view's entries 0 .. n - 1.
+// With staged, only one of launch_export and launch_export_to_rec + launch_rec_to_view does the work.
+void launch_export(State src, int64_t n_res, const void *view, int64_t off, const DevMaterial *mats, int aux,
+                   const uint32_t *staged, hipStream_t s);
+// want: the kAux* channels to put into the records
+void launch_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux, int want, float *rec,
+                          const uint32_t *staged, hipStream_t s);
+void launch_rec_to_view(const float *rec, const void *view, int64_t off, const uint32_t *staged, hipStream_t s);
 // Particle volume dx^3 / (particles in the cell) and mass rho vol into caller buffers
 // (one channel each, ZMPM_LAYOUT_*) at the caller particle index; cnt: scratch of 64
 // words per grid block.
@@ -352,8 +373,9 @@ void launch_particle_beta(State A, int64_t n, Lattice L, const DevMaterial *mats
 // permutation of every channel of src into dst by order (dst[k] = src[order[k]]).
 void launch_morton_codes(int32_t layout, int32_t nch, int64_t n, const float *src, int32_t x_chn, const float lo[3],
                          const float ext[3], uint32_t *codes, hipStream_t s);
+// rec: scratch of 32 floats per particle for the way through records (null: directly), staged: one word
 void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float *src, float *dst,
-                             const uint32_t *order, hipStream_t s);
+                             const uint32_t *order, float *rec, uint32_t *staged, hipStream_t s);
 
 struct VolumeOut {
     int32_t layout, tile_channels;
