@@ -25,6 +25,8 @@
 #include "mpm_device.h"
 #include "../../include/zmpm.h"
 
+#include <type_traits>
+
 namespace zmpm {
 
 namespace {
@@ -1846,7 +1848,7 @@ constexpr uint32_t kDirStay = 13;
 // in LDS only when it lists a particle, and a block segment that lists none
 // takes its ranks from the particle order without ballots.  Every direction
 // equals the one the full interpolation gives.
-// NT: threads per workgroup (64 or 256; picked per context by zmpm_autotune).
+// NT: threads per workgroup (64 or 256; the context's rule or zmpm_autotune).
 // AFLIP: the FLIP transfers (grid velocities v and vstar, the particle's own v
 // blended in, the particle's beta or 0 for non-affine FLIP); every particle is
 // interpolated.
@@ -2696,11 +2698,11 @@ __global__ void __launch_bounds__(kThreads) k_import(State dst, zmpm_particles v
 // A permutation of particles whose channels lie in planes or tiles reads (or writes) four bytes of a
 // cache line per particle and channel when the order is far from the memory's.  Such a one goes
 // through records instead: kRec floats of a particle in one 128-byte line.  One pass turns channels
-// into records, coalesced on both sides through LDS; the permuted side moves whole lines.  That
-// doubles the bytes (4.9 million particles of 256 scenes: export 1,936 -> 238 + 261 us, at 5 TB/s; a
-// shuffled 613,057: import and sort by 35 + 27 us for 48 + 240), so an order that is local (runs of a wave's 64 entries in few lines) keeps the
-// direct kernels.  k_order_sample decides on the device, without a synchronisation: both kinds are
-// launched and one returns at once.
+// into records, coalesced on both sides through LDS; the permuted side moves whole lines.  Export of
+// 4.9 million particles of 256 scenes: 1,936 -> 238 + 261 us, at 5 TB/s; import and permutation of a
+// shuffled 613,057: 48 + 240 -> 35 + 27 us.  It doubles the bytes, so an order that is local (runs of
+// a wave's 64 entries in few lines) keeps the direct kernels.  k_order_sample decides on the device,
+// without a synchronisation: both kinds are launched and one returns at once.
 constexpr int kRec = 32;
 constexpr int kRecPitch = 36;  // floats of a record's row in LDS: 16-byte rows on distinct banks
 constexpr int kRecWaves = kThreads / 64;
@@ -3380,17 +3382,17 @@ void launch_stress(State A, int64_t n, Lattice L, const DevMaterial *mats, float
         hipLaunchKernelGGL(k_stress<false>, dim3(grid_for(n, 2048)), dim3(kThreads), 0, s, A, n, L, mats, sig, stride);
 }
 
-// P2G over `units` parts, the host's estimate (the count + 25 % + 64): k_p2g_wide while the count is
-// at most the chip's 256 CUs, where its shorter chain is the launch's time (figures at the kernel),
-// k_p2g above.  The two give the same bits.
-constexpr int64_t kWideMaxUnits = 384;
+// P2G over about `parts` parts (max_blocks: the bound that sizes the grid): k_p2g_wide up to the
+// chip's 256 CUs, where its shorter chain is the launch's time (figures at the kernel), k_p2g above.
+// The two give the same bits.
+constexpr int64_t kWideMaxParts = 256;
 template <int MODE>
-void launch_p2g_mode(int64_t units, hipStream_t s, State A, Partition P, Lattice L, const DevMaterial *mats,
+void launch_p2g_mode(int64_t parts, int64_t max_blocks, hipStream_t s, State A, Partition P, Lattice L, const DevMaterial *mats,
                      const float *sig, int64_t stride, float *tiles, DevStatus *st, AdjScatter adj,
                      uint32_t skip_upto) {
-    const dim3 g(persistent_grid(units, 1, 1 << 20));
+    const dim3 g(persistent_grid(max_blocks, 1, 1 << 20));
     constexpr bool CAN_PP = MODE != kP2GAdjoint;
-    if (skip_upto == 0u && units <= kWideMaxUnits) {
+    if (skip_upto == 0u && parts <= kWideMaxParts) {
         if (CAN_PP && L.pp_mass)
             hipLaunchKernelGGL((k_p2g_wide<MODE, CAN_PP>), g, dim3(kWideThreads), 0, s, A, P, L, mats, sig, stride,
                                tiles, st, adj);
@@ -3407,13 +3409,14 @@ void launch_p2g_mode(int64_t units, hipStream_t s, State A, Partition P, Lattice
 }
 
 void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
-                float *tiles, DevStatus *st, int64_t max_blocks, hipStream_t s, bool sparse, bool flush) {
+                float *tiles, DevStatus *st, int64_t parts, int64_t max_blocks, hipStream_t s, bool sparse,
+                bool flush) {
     if (max_blocks <= 0) return;
     const dim3 g(persistent_grid(max_blocks, 1, 1 << 20));
     // with sparse, blocks of <= kSparseMax particles go to the one-wave kernel (one chunk either way)
     const uint32_t skip = sparse ? (uint32_t)kSparseMax : 0u;
     if (!flush)
-        launch_p2g_mode<kP2GForward>(max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, skip);
+        launch_p2g_mode<kP2GForward>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, skip);
     else if (L.pp_mass)
         hipLaunchKernelGGL((k_p2g<kP2GForward, true, true>), g, dim3(kP2GThreads), 0, s, A, P, L, mats, sig, stride,
                            tiles, st, AdjScatter{}, skip);
@@ -3426,17 +3429,19 @@ void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const 
 }
 
 void launch_p2g_aflip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
-                      float *tiles, float *tiles2, DevStatus *st, int64_t max_blocks, hipStream_t s) {
+                      float *tiles, float *tiles2, DevStatus *st, int64_t parts, int64_t max_blocks,
+                      hipStream_t s) {
     if (max_blocks <= 0) return;
-    launch_p2g_mode<kP2GMomentum>(max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
-    launch_p2g_mode<kP2GStress>(max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GMomentum>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GStress>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
 }
 
 void launch_p2g_flip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
-                     float *tiles, float *tiles2, DevStatus *st, int64_t max_blocks, hipStream_t s) {
+                     float *tiles, float *tiles2, DevStatus *st, int64_t parts, int64_t max_blocks,
+                     hipStream_t s) {
     if (max_blocks <= 0) return;
-    launch_p2g_mode<kP2GFlipMomentum>(max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
-    launch_p2g_mode<kP2GFlipStress>(max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GFlipMomentum>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
+    launch_p2g_mode<kP2GFlipStress>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
 }
 
 void launch_grid_aflip(int mode, Partition P, Lattice L, const float *tiles, const float *tiles2, float *grid,
@@ -3447,10 +3452,10 @@ void launch_grid_aflip(int mode, Partition P, Lattice L, const float *tiles, con
                        tiles, tiles2, grid, gstar, gvmax, vclear, nclear);
 }
 
-void launch_p2g_adjoint(State A, Partition P, Lattice L, AdjScatter adj, float *tiles, DevStatus *st,
+void launch_p2g_adjoint(State A, Partition P, Lattice L, AdjScatter adj, float *tiles, DevStatus *st, int64_t parts,
                         int64_t max_blocks, hipStream_t s) {
     if (max_blocks <= 0) return;
-    launch_p2g_mode<kP2GAdjoint>(max_blocks, s, A, P, L, nullptr, nullptr, 0, tiles, st, adj, 0u);
+    launch_p2g_mode<kP2GAdjoint>(parts, max_blocks, s, A, P, L, nullptr, nullptr, 0, tiles, st, adj, 0u);
 }
 
 void launch_grid(int mode, Partition P, Lattice L, const float *tiles, float *grid, float *gvmax,
@@ -3466,24 +3471,28 @@ void launch_reduce_vmax(const float *gvmax, Partition P, int64_t max_blocks, uin
                        (const uint32_t *)P.gblk_scene, (const uint32_t *)P.counts, out);
 }
 
+using I64 = std::integral_constant<int, 64>;
+using I256 = std::integral_constant<int, 256>;
+using I512 = std::integral_constant<int, 512>;
+
 void launch_g2p_move(State A, Partition P, Lattice L, const float *grid, const float *gvmax, Binning B,
                      DevStatus *st, int64_t max_blocks, hipStream_t s, int wg, const float *gstar, bool nonaffine,
                      bool fused) {
     if (max_blocks <= 0) return;
     const dim3 g(persistent_grid(max_blocks, 1, 1 << 20));
-    const int na = nonaffine ? 1 : 0;
-    if (gstar)
-        hipLaunchKernelGGL((k_g2p_move<64, true>), g, dim3(64), 0, s, A, P, L, grid, gvmax, B, st, gstar, na);
-    else if (fused && wg == 64)
-        hipLaunchKernelGGL((k_g2p_move<64, false, true>), g, dim3(64), 0, s, A, P, L, grid, gvmax, B, st, gstar, na);
-    else if (fused)
-        hipLaunchKernelGGL((k_g2p_move<kThreads, false, true>), g, dim3(kThreads), 0, s, A, P, L, grid, gvmax, B, st,
-                           gstar, na);
-    else if (wg == 64)
-        hipLaunchKernelGGL((k_g2p_move<64, false>), g, dim3(64), 0, s, A, P, L, grid, gvmax, B, st, gstar, na);
-    else
-        hipLaunchKernelGGL((k_g2p_move<kThreads, false>), g, dim3(kThreads), 0, s, A, P, L, grid, gvmax, B, st,
-                           gstar, na);
+    auto launch = [&](auto nt, auto aflip, auto fuse) {
+        constexpr int NT = decltype(nt)::value;
+        hipLaunchKernelGGL((k_g2p_move<NT, decltype(aflip)::value, decltype(fuse)::value>), g, dim3(NT), 0, s, A, P, L,
+                           grid, gvmax, B, st, gstar, nonaffine ? 1 : 0);
+    };
+    auto by_size = [&](auto aflip) {
+        if (wg == 64) launch(I64{}, aflip, std::false_type{});
+        else launch(I256{}, aflip, std::false_type{});
+    };
+    if (fused && wg == 64) launch(I64{}, std::false_type{}, std::true_type{});
+    else if (fused) launch(I256{}, std::false_type{}, std::true_type{});
+    else if (gstar) by_size(std::true_type{});
+    else by_size(std::false_type{});
 }
 
 void launch_g2p2g(State A, State Bst, Partition P, Partition Pn, Lattice L, const float *grid, Binning Bn,
@@ -3576,16 +3585,19 @@ void launch_g2p_update(bool scatter, State A, State Bst, Partition P, Partition 
     u.aux = aux;
     u.nonaffine = nonaffine ? 1 : 0;
     const unsigned g = persistent_grid(max_blocks, 1, 1 << 20);
-    if (gstar && scatter)
-        hipLaunchKernelGGL((k_g2p_update<true, 64, true>), dim3(g), dim3(64), 0, s, u);
-    else if (gstar)
-        hipLaunchKernelGGL((k_g2p_update<false, 64, true>), dim3(g), dim3(64), 0, s, u);
-    else if (scatter && wg == 64)
-        hipLaunchKernelGGL((k_g2p_update<true, 64>), dim3(g), dim3(64), 0, s, u);
-    else if (scatter)
-        hipLaunchKernelGGL((k_g2p_update<true, kThreads>), dim3(g), dim3(kThreads), 0, s, u);
-    else
-        hipLaunchKernelGGL((k_g2p_update<false, kThreads>), dim3(g), dim3(kThreads), 0, s, u);
+    auto launch = [&](auto scat, auto nt, auto aflip) {
+        constexpr int NT = decltype(nt)::value;
+        hipLaunchKernelGGL((k_g2p_update<decltype(scat)::value, NT, decltype(aflip)::value>), dim3(g), dim3(NT), 0, s, u);
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (gstar && scatter && wg == 64) launch(Yes{}, I64{}, Yes{});
+    else if (gstar && scatter) launch(Yes{}, I256{}, Yes{});
+    else if (gstar) launch(No{}, I256{}, Yes{});
+    else if (scatter && wg == 64) launch(Yes{}, I64{}, No{});
+    else if (scatter && wg == 512) launch(Yes{}, I512{}, No{});
+    else if (scatter) launch(Yes{}, I256{}, No{});
+    else launch(No{}, I256{}, No{});
 }
 
 void launch_import(State dst, const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, DevStatus *st,

@@ -68,15 +68,39 @@ struct zmpm_ctx {
     int64_t n = 0;
     bool partitioned = false;  // the partition describes the current particle positions
     bool loaded_sorted = false;  // the resident state was loaded from a save (saves are block-sorted)
-    int wg_move = 256, wg_update = 256;  // G2P workgroup sizes (zmpm_autotune)
+    // the particle block parts of the last partition the host knows of (a captured graph keeps the
+    // kernels that its capture chose: every variant gives the same bits for any count)
+    int64_t parts_now() const {
+        const volatile uint32_t *c = host_counts;
+        return c && c[0] ? (int64_t)c[0] + c[2] : max_units();
+    }
+    // Threads per workgroup (one part each) of the G2P kernels: as zmpm_autotune found, else by how
+    // many parts there are.  Few leave wave slots empty, so a part gets as many threads as pay; many
+    // fill the chip with one wave each, which waits at no barrier.
+    // Move, 180 parts of 363 particles: 13.8 us with 64 threads, 9.9 with 256, 9.4 with 512; 1,180 of
+    // 340: 16.2, 11.7, 18.0; 1,800 of 340: 16.9, 18.9, 25.3; 9,990 of 420: 48, 71, 131; 82,757 of 60:
+    // 207, 345, -.  Update, the same: 22.2, 12.2, 10.5; 27.2, 19.2, 22.2; 27.1, 26.8, 32.3; 128, 124,
+    // 160; 375, 517, -; about 400 parts: 24.1, 13.5, 12.1; 740: 26.1, 16.4, 19.1.
+    // FLIP transfers (the particles are all interpolated, twice the registers), move and update, 366
+    // parts: 27 and 51 with 64, 16 and 22 with 256, 15 and 24 with 512; 1,750: 37 and 46, 29 and 47, 35
+    // and 58; 5,800: 88 and 176, 68 and 156, 97 and 183.
+    int wg_move_tuned = 0, wg_update_tuned = 0;
+    bool many_small_parts() const { return parts_now() >= 1536 && n <= 96 * parts_now(); }
+    int wg_move() const {
+        if (wg_move_tuned) return wg_move_tuned;
+        return (flip_style() ? many_small_parts() : parts_now() >= 1536) ? 64 : 256;
+    }
+    int wg_update() const {
+        if (wg_update_tuned == 64 || (!wg_update_tuned && many_small_parts())) return 64;
+        return !flip_style() && parts_now() <= 512 ? 512 : 256;
+    }
     // one-wave P2G for blocks of <= 64 particles, a launch of its own: as zmpm_autotune found, else
     // where the chip is full of blocks that hold few particles.  (A launch that finds no such block
     // still costs 13-18 us; on 82,757 blocks of 60 particles on average it gains 423 against 440 us.)
     int p2g_sparse_tuned = -1;
     bool p2g_sparse() const {
         if (p2g_sparse_tuned >= 0) return p2g_sparse_tuned != 0;
-        const int64_t np = host_counts ? (int64_t)((volatile uint32_t *)host_counts)[0] : 0;
-        return np >= 16384 && n <= 96 * np;
+        return parts_now() >= 16384 && n <= 96 * parts_now();
     }
     bool fuse = false;                   // APIC: the fused G2P / P2G pass (zmpm_autotune, zmpm_set_fused);
                                          // while on, every P2G of the context uses its chunk-flush grouping
@@ -796,15 +820,16 @@ int32_t zmpm_p2g(zmpm_ctx *ctx, float dt) {
         if (ctx->flip_style()) {
             if (ctx->transfer == ZMPM_TRANSFER_FLIP)
                 launch_p2g_flip(ctx->st[ctx->cur], ctx->part[ctx->pcur], ctx->L, ctx->mats, ctx->sig, ctx->cap,
-                                ctx->tiles, ctx->tiles2, ctx->status, ctx->max_units(), ctx->stream);
+                                ctx->tiles, ctx->tiles2, ctx->status, ctx->parts_now(), ctx->max_units(), ctx->stream);
             else
                 launch_p2g_aflip(ctx->st[ctx->cur], ctx->part[ctx->pcur], ctx->L, ctx->mats, ctx->sig, ctx->cap,
-                                 ctx->tiles, ctx->tiles2, ctx->status, ctx->max_units(), ctx->stream);
+                                 ctx->tiles, ctx->tiles2, ctx->status, ctx->parts_now(), ctx->max_units(), ctx->stream);
             launch_grid_aflip(GRID_COMBINE, ctx->part[ctx->pcur], ctx->L, ctx->tiles, ctx->tiles2, ctx->grid,
                               ctx->gstar, ctx->gvmax, ctx->max_gblocks(), ctx->stream);
         } else {
             launch_p2g(ctx->st[ctx->cur], ctx->part[ctx->pcur], ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles,
-                       ctx->status, ctx->max_units(), ctx->stream, ctx->p2g_sparse(), ctx->fused_path());
+                       ctx->status, ctx->parts_now(), ctx->max_units(), ctx->stream, ctx->p2g_sparse(),
+                       ctx->fused_path());
             launch_grid(GRID_COMBINE, ctx->part[ctx->pcur], ctx->L, ctx->tiles, ctx->grid, ctx->gvmax,
                         ctx->max_gblocks(), ctx->stream);
         }
@@ -1139,12 +1164,12 @@ void substep_fused(zmpm_ctx *ctx, hipEvent_t *ev, int grow, bool last) {
     const State A = ctx->st[ctx->cur], B = ctx->st[ctx->cur ^ 1];
     const Partition P = ctx->part[ctx->pcur], Pn = ctx->part[ctx->pcur ^ 1];
     const int grid_mode = GRID_COMBINE | GRID_UPDATE | GRID_BOUNDARY;
-    const int64_t npb = ctx->max_pblocks() << grow, ngb = ctx->max_gblocks() << grow;
+    const int64_t np = ctx->parts_now(), npb = ctx->max_pblocks() << grow, ngb = ctx->max_gblocks() << grow;
     if (ev) HIP_CHECK(hipEventRecord(ev[0], s));
     if (!ctx->tiles_valid) launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, ctx->stress_general());
     if (ev) HIP_CHECK(hipEventRecord(ev[1], s));
     if (!ctx->tiles_valid)
-        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, npb, s, ctx->p2g_sparse(), true);
+        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, ctx->p2g_sparse(), true);
     if (ev) HIP_CHECK(hipEventRecord(ev[2], s));
     launch_grid(grid_mode, P, ctx->L, ctx->tiles, ctx->grid, ctx->gvmax, ngb, s, nullptr, ctx->vmax, ctx->L.nscenes);
     launch_colliders(P, ctx->L, ctx->grid, ctx->gvmax, ngb, true, s);
@@ -1152,7 +1177,7 @@ void substep_fused(zmpm_ctx *ctx, hipEvent_t *ev, int grow, bool last) {
     if (ctx->cols_move) launch_step_colliders(ctx->L, -1.0f, s);
     if (ev) HIP_CHECK(hipEventRecord(ev[3], s));
     // the move pass also reduces this substep's MaxVelSqr (ctx->bin.vmax_out)
-    launch_g2p_move(A, P, ctx->L, ctx->grid, ctx->gvmax, ctx->bin, ctx->status, npb, s, ctx->wg_move, nullptr, false,
+    launch_g2p_move(A, P, ctx->L, ctx->grid, ctx->gvmax, ctx->bin, ctx->status, npb, s, ctx->wg_move(), nullptr, false,
                     true);
     if (ev) HIP_CHECK(hipEventRecord(ev[4], s));
     launch_lattice_scan(ctx->L, Pn, ctx->bin, P.tile_used, ctx->n, ctx->status, s);
@@ -1190,8 +1215,8 @@ void fused_prologue(zmpm_ctx *ctx, bool force = false) {
     const State A = ctx->st[ctx->cur];
     const Partition P = ctx->part[ctx->pcur];
     launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->stream, ctx->stress_general());
-    launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, ctx->max_units(), ctx->stream,
-               ctx->p2g_sparse(), true);
+    launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, ctx->parts_now(), ctx->max_units(),
+               ctx->stream, ctx->p2g_sparse(), true);
     ctx->tiles_valid = true;
 }
 
@@ -1205,7 +1230,7 @@ void substep_once(zmpm_ctx *ctx, hipEvent_t *ev, int grow = 0, bool last = true)
     const Partition P = ctx->part[ctx->pcur], Pn = ctx->part[ctx->pcur ^ 1];
     const int grid_mode = GRID_COMBINE | GRID_UPDATE | GRID_BOUNDARY;
     // P2G and both G2P passes work per part
-    const int64_t npb = ctx->max_units() << grow, ngb = ctx->max_gblocks() << grow;
+    const int64_t np = ctx->parts_now(), npb = ctx->max_units() << grow, ngb = ctx->max_gblocks() << grow;
     ctx->tiles_valid = false;
     if (ev) HIP_CHECK(hipEventRecord(ev[0], s));
     launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, ctx->stress_general());
@@ -1214,11 +1239,11 @@ void substep_once(zmpm_ctx *ctx, hipEvent_t *ev, int grow = 0, bool last = true)
     const bool aflip = ctx->flip_style(), nonaffine = ctx->transfer == ZMPM_TRANSFER_FLIP;
     float *gstar = aflip ? ctx->gstar : nullptr;
     if (nonaffine)
-        launch_p2g_flip(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->tiles2, ctx->status, npb, s);
+        launch_p2g_flip(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->tiles2, ctx->status, np, npb, s);
     else if (aflip)
-        launch_p2g_aflip(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->tiles2, ctx->status, npb, s);
+        launch_p2g_aflip(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->tiles2, ctx->status, np, npb, s);
     else
-        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, npb, s, ctx->p2g_sparse());
+        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, ctx->p2g_sparse());
     if (ev) HIP_CHECK(hipEventRecord(ev[2], s));
     if (aflip)
         launch_grid_aflip(grid_mode, P, ctx->L, ctx->tiles, ctx->tiles2, ctx->grid, gstar, ctx->gvmax, ngb, s,
@@ -1233,7 +1258,7 @@ void substep_once(zmpm_ctx *ctx, hipEvent_t *ev, int grow = 0, bool last = true)
     // G2P pass 1: direction of every particle's new block, per-block counts, destination marks, and
     // UpdateZSGrid's MaxVelSqr output of this substep (MPMPipeline.cu:939-942) per scene on the
     // device, into the words k_grid cleared
-    launch_g2p_move(A, P, ctx->L, ctx->grid, ctx->gvmax, ctx->bin, ctx->status, npb, s, ctx->wg_move, gstar,
+    launch_g2p_move(A, P, ctx->L, ctx->grid, ctx->gvmax, ctx->bin, ctx->status, npb, s, ctx->wg_move(), gstar,
                     nonaffine);
     if (ev) HIP_CHECK(hipEventRecord(ev[4], s));
     // the next partition: particle blocks, their first particles, grid blocks
@@ -1241,7 +1266,7 @@ void substep_once(zmpm_ctx *ctx, hipEvent_t *ev, int grow = 0, bool last = true)
     ctx->psize[ctx->pcur ^ 1] = ctx->L.part_shift;
     if (ev) HIP_CHECK(hipEventRecord(ev[5], s));
     // G2P pass 2: full update, written straight into the next stable block order
-    launch_g2p_update(true, A, B, P, Pn, ctx->L, ctx->grid, ctx->bin, npb, s, ctx->wg_update, gstar, ctx->aux(),
+    launch_g2p_update(true, A, B, P, Pn, ctx->L, ctx->grid, ctx->bin, npb, s, ctx->wg_update(), gstar, ctx->aux(),
                       nonaffine);
     if (ctx->has_plastic) launch_return_mapping(B, ctx->n, ctx->mats, s);  // ZSReturnMapping after G2P
     if (ev) HIP_CHECK(hipEventRecord(ev[6], s));
@@ -1348,8 +1373,8 @@ int32_t zmpm_autotune(zmpm_ctx *ctx, const zmpm_step_params *p, int32_t nsteps, 
             int pick = 0;
             for (int k = 0; k < ncand; ++k) {
                 if (k == 4) cand[4] = Cand{cand[pick].move, cand[pick].update, 0, 0};
-                ctx->wg_move = cand[k].move;
-                if (!cand[k].fuse) ctx->wg_update = cand[k].update;
+                ctx->wg_move_tuned = cand[k].move;
+                if (!cand[k].fuse) ctx->wg_update_tuned = cand[k].update;
                 ctx->p2g_sparse_tuned = cand[k].sparse;
                 ctx->fuse = cand[k].fuse != 0;
                 HIP_CHECK(hipMemcpyAsync(ctx->st[ctx->cur].ch, saved, sizeof(float) * state_floats(ctx->n),
@@ -1369,8 +1394,8 @@ int32_t zmpm_autotune(zmpm_ctx *ctx, const zmpm_step_params *p, int32_t nsteps, 
                     pick = k;
                 }
             }
-            ctx->wg_move = cand[pick].move;
-            if (!cand[pick].fuse) ctx->wg_update = cand[pick].update;
+            ctx->wg_move_tuned = cand[pick].move;
+            if (!cand[pick].fuse) ctx->wg_update_tuned = cand[pick].update;
             ctx->p2g_sparse_tuned = cand[pick].sparse;
             ctx->fuse = cand[pick].fuse != 0;
             HIP_CHECK(hipMemcpyAsync(ctx->st[ctx->cur].ch, saved, sizeof(float) * state_floats(ctx->n),
@@ -1380,8 +1405,8 @@ int32_t zmpm_autotune(zmpm_ctx *ctx, const zmpm_step_params *p, int32_t nsteps, 
             full_partition(ctx);
             HIP_CHECK(hipStreamSynchronize(ctx->stream));
             if (choice) {
-                choice[0] = ctx->wg_move;
-                choice[1] = ctx->fused_path() ? 0 : ctx->wg_update;
+                choice[0] = ctx->wg_move_tuned;
+                choice[1] = ctx->fused_path() ? 0 : ctx->wg_update_tuned;
                 choice[2] = ctx->p2g_sparse_tuned;
             }
         } catch (...) {
@@ -1531,11 +1556,11 @@ int32_t zmpm_adjoint_substep(zmpm_ctx *ctx, const zmpm_step_params *p, const zmp
         hipStream_t s = ctx->stream;
         const State A = ctx->st[ctx->cur];
         const Partition P = ctx->part[ctx->pcur];
-        const int64_t npb = ctx->max_units(), ngb = ctx->max_gblocks();
+        const int64_t np = ctx->parts_now(), npb = ctx->max_units(), ngb = ctx->max_gblocks();
         AdjArrays aa{adj->x, adj->v, adj->C, adj->F, adj->mu, adj->lam, adj->n};
         // forward transfer again: combined mass and momentum in grid, updated velocities in grid_v
         launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, ctx->stress_general());
-        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, npb, s, ctx->p2g_sparse(),
+        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, ctx->p2g_sparse(),
                    ctx->fused_path());
         launch_grid(GRID_COMBINE | GRID_KEEP | GRID_UPDATE | GRID_BOUNDARY, P, ctx->L, ctx->tiles, ctx->grid,
                     ctx->gvmax, ngb, s, ctx->grid_v);
@@ -1543,7 +1568,7 @@ int32_t zmpm_adjoint_substep(zmpm_ctx *ctx, const zmpm_step_params *p, const zmp
         const int64_t stride = ctx->cap;
         launch_g2p_adjoint(A, P, ctx->L, ctx->grid_v, aa, ctx->pay, ctx->pay + 3 * stride, stride, npb, s);
         launch_p2g_adjoint(A, P, ctx->L, AdjScatter{ctx->pay, ctx->pay + 3 * stride, stride}, ctx->tiles,
-                           ctx->status, npb, s);
+                           ctx->status, np, npb, s);
         launch_grid(GRID_COMBINE, P, ctx->L, ctx->tiles, ctx->gbar, ctx->gvmax, ngb, s);
         launch_grid_adjoint(P, ctx->L, ctx->grid, ctx->gbar, ngb, s);
         launch_p2g_gather_adjoint(A, P, ctx->L, ctx->mats, ctx->gbar, aa, npb, s);

@@ -237,7 +237,7 @@ struct AdjScatter {
     int64_t stride;
 };
 // Adjoint of G2P's velocity gather: tiles receive sum_p W (a_p + B_p d) per node (mass channel 0).
-void launch_p2g_adjoint(State A, Partition P, Lattice L, AdjScatter adj, float *tiles, DevStatus *st,
+void launch_p2g_adjoint(State A, Partition P, Lattice L, AdjScatter adj, float *tiles, DevStatus *st, int64_t parts,
                         int64_t max_blocks, hipStream_t s);
 // Adjoint arrays of a differentiated substep, by caller particle index: planes of n
 // entries x (3), v (3), C (9), F (9; J-fluid: F[0] = dL/dJ); mu, lam accumulate dL/dmu, dL/dlam.
@@ -255,10 +255,11 @@ void launch_p2g_gather_adjoint(State A, Partition P, Lattice L, const DevMateria
 void launch_stress(State A, int64_t n, Lattice L, const DevMaterial *mats, float *sig, int64_t stride,
                    hipStream_t s, bool general = true);
 // P2G of every particle block into its tile (fixed-corotated stress terms from launch_stress).
+// parts: how many the host believes there are (chooses the kernel), max_blocks: sizes the grid.
 // sparse: blocks of at most 64 particles go to a one-wave-per-block kernel (a second launch).
 // flush: the fused pass's chunk-flush grouping of blocks of more than one chunk (k_p2g FLUSH)
 void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
-                float *tiles, DevStatus *st, int64_t max_blocks, hipStream_t s, bool sparse = false,
+                float *tiles, DevStatus *st, int64_t parts, int64_t max_blocks, hipStream_t s, bool sparse = false,
                 bool flush = false);
 // mode bits for launch_grid
 enum { GRID_COMBINE = 1, GRID_UPDATE = 2, GRID_BOUNDARY = 4, GRID_CLEAR = 8, GRID_KEEP = 16 };
@@ -300,10 +301,12 @@ void launch_g2p_update(bool scatter, State A, State B, Partition P, Partition Pn
 // Affine FLIP transfers: P2G of the momentum (into tiles) and of the stress
 // (into tiles2), and their grid stages (grid: m, v; gstar: m, vstar).
 void launch_p2g_aflip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
-                      float *tiles, float *tiles2, DevStatus *st, int64_t max_blocks, hipStream_t s);
+                      float *tiles, float *tiles2, DevStatus *st, int64_t parts, int64_t max_blocks,
+                      hipStream_t s);
 // FLIP transfer: P2G of W m v (into tiles) and of W (-dt vol P F^T grad W) (into tiles2).
 void launch_p2g_flip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
-                     float *tiles, float *tiles2, DevStatus *st, int64_t max_blocks, hipStream_t s);
+                     float *tiles, float *tiles2, DevStatus *st, int64_t parts, int64_t max_blocks,
+                     hipStream_t s);
 void launch_grid_aflip(int mode, Partition P, Lattice L, const float *tiles, const float *tiles2, float *grid,
                        float *gstar, float *gvmax, int64_t max_blocks, hipStream_t s, uint32_t *vclear = nullptr,
                        int32_t nclear = 0);
