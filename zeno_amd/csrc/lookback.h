@@ -19,6 +19,10 @@ namespace zmpm {
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanThreads * kScanItems;  // 4096
+constexpr int kSmallScanItems = 4;                    // per thread, for a scan of few tiles
+constexpr int kSmallScanTiles = 64;
+constexpr int64_t kSmallScanTile = kScanThreads * kSmallScanItems;  // 1024
+inline bool small_scan(int64_t n) { return n <= kSmallScanTiles * kSmallScanTile; }
 constexpr uint64_t kScanValueMask = (1ull << 62) - 1;
 constexpr uint64_t kScanFlagAgg = 1ull << 62;
 constexpr uint64_t kScanFlagPrefix = 2ull << 62;
@@ -76,29 +80,6 @@ __device__ __forceinline__ uint64_t lookback_wave(const ScanState &S, uint32_t t
                                __HIP_MEMORY_SCOPE_AGENT);
     }
     return excl;
-}
-
-// Exclusive scan of one 64-bit value per thread across the 256-thread block.
-__device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, uint64_t *s_wave, uint64_t *total) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    uint64_t inc = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint64_t y = __shfl_up(inc, off, 64);
-        if (lane >= off) inc += y;
-    }
-    if (lane == 63) s_wave[w] = inc;
-    __syncthreads();
-    uint64_t pre = 0, tot = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint64_t s = s_wave[k];
-        pre += (k < w) ? s : 0ull;
-        tot += s;
-    }
-    __syncthreads();
-    *total = tot;
-    return pre + inc - v;
 }
 
 }  // namespace zmpm

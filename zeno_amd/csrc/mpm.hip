@@ -139,47 +139,76 @@ __global__ void __launch_bounds__(kThreads) k_mark_blocks(const uint32_t *skeys,
     }
 }
 
+// Inclusive sum over the wave's lanes by DPP row shifts and broadcasts.
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
 // Lattice scan: two decoupled look-back chains over the lattice in index
 // order give every marked entry its particle-block id (and the first
 // particle of that block, from the per-block particle counts) and its
-// grid-block id.  Clears the marks and counts it read.  A tile of 4096 entries
-// is read and written only if it may hold a new mark or holds an entry of this
-// partition buffer's previous contents (Pn.tile_used); otherwise it contributes
-// zero and its entries are already -1, so a sparse lattice costs its occupied
-// tiles, not its size.  New marks lie within B.mark_radius tiles of a tile
+// grid-block id.  Clears the marks and counts it read.
+// SMALL: a lattice of at most kSmallScanTiles tiles of four entries a thread, every one visited.
+// Otherwise a tile of 4096 entries is read and written only if it may hold a new
+// mark or holds an entry of this partition buffer's previous contents
+// (Pn.tile_used); if not, it contributes zero and its entries are already -1, so a
+// sparse lattice costs its occupied tiles, not its size.  New marks lie within
+// B.mark_radius tiles of a tile
 // holding a block of the partition the particles move from (prev_used; a
 // block marks entries at offsets -1 .. +2 per axis), or anywhere when
 // B.tile_mark forces a tile (full re-bin).  Entries move as 16-byte vectors.
 // The grid-block chain also counts extra parts (bits 32-61: a particle block of d
 // particles has ceil(d / 2^L.part_shift) - 1 of them), so every block gets the number of
 // extra parts before it and every extra part its block and first particle.
+// The launch is a chain of dependent latencies (tile, entries, scan, look-back, entries), so the loads
+// of one step go out together, the scans are DPP adds and a lattice of at most 64 tiles takes them by
+// workgroup number.  1,331 entries: 8.1 -> 3.6 us, 42,875: 9.7 -> 4.7, 8 scenes: 11.7 -> 5.4, 300,763:
+// 12.2 -> 10.8, 256 scenes of 6.4 million (a tile finds its scene with the whole wave): 94 -> 60.
+// Tiles by workgroup number: the 64 workgroups that may wait never fill the chip (2,048 places), so
+// the one they wait for always gets a place; more tiles take a ticket.
 __device__ __forceinline__ uint32_t extra_parts(uint32_t d, uint32_t shift) { return d == 0u ? 0u : (d - 1u) >> shift; }
 
+template <bool SMALL>
 __global__ void __launch_bounds__(kScanThreads) k_lattice_scan(Lattice L, Partition Pn, Binning B,
-                                                              const uint32_t *prev_used, DevStatus *st) {
-    __shared__ uint64_t s_wave[4];
+                                                              const uint32_t *prev_used) {
+    constexpr int ITEMS = SMALL ? kSmallScanItems : kScanItems;
+    constexpr int NWAVE = kScanThreads / 64;
+    __shared__ uint32_t s_sum[3][NWAVE];
     __shared__ uint32_t s_tile;
+    __shared__ uint64_t s_pref[2];
     // particle-block count in the low kPBlkBits bits (blocks <= capacity < 2^27), particles above
     constexpr uint64_t kBlkMask = (1ull << kPBlkBits) - 1;
-    if (threadIdx.x == 0) s_tile = atomicAdd(B.scan_p.tile_ctr, 1u);
-    __syncthreads();
-    const uint32_t tile = s_tile;
-    const int64_t size = L.size;
-    uint32_t near = B.tile_mark[tile] | Pn.tile_used[tile];
-    {
-        const int64_t lo = (int64_t)tile - B.mark_radius, hi = (int64_t)tile + B.mark_radius;
-        for (int64_t q = lo < 0 ? 0 : lo; q <= hi && q < B.scan_tiles; ++q) near |= prev_used[q];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t tile = blockIdx.x;
+    if (!SMALL && B.scan_tiles > kSmallScanTiles) {
+        if (threadIdx.x == 0) s_tile = atomicAdd(B.scan_p.tile_ctr, 1u);
+        __syncthreads();
+        tile = s_tile;
     }
-    const bool need = near != 0u;
-    const int64_t base = (int64_t)tile * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    const bool full = base + kScanItems <= size;
-    uint32_t f[kScanItems], d[kScanItems];
+    const int64_t size = L.size;
+    bool need = true;
+    if (!SMALL) {
+        uint32_t near = lane == 0 ? B.tile_mark[tile] | Pn.tile_used[tile] : 0u;
+        const int64_t lo = (int64_t)tile - B.mark_radius;
+        const int64_t hi = min((int64_t)tile + B.mark_radius, B.scan_tiles - 1);
+        for (int64_t q = max(lo, (int64_t)0) + lane; q <= hi; q += 64) near |= prev_used[q];
+        need = __ballot(near != 0u) != 0ull;  // every wave sees all of them
+    }
+    const int64_t base = ((int64_t)tile * kScanThreads + threadIdx.x) * ITEMS;
+    const bool full = base + ITEMS <= size;
+    uint32_t f[ITEMS], d[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) f[k] = d[k] = 0u;
+    for (int k = 0; k < ITEMS; ++k) f[k] = d[k] = 0u;
     if (need) {
         if (full) {
 #pragma unroll
-            for (int q = 0; q < kScanItems / 4; ++q) {
+            for (int q = 0; q < ITEMS / 4; ++q) {
                 const uint4 fv = *reinterpret_cast<const uint4 *>(B.lat_flag + base + 4 * q);
                 const uint4 dv = *reinterpret_cast<const uint4 *>(B.dcount + base + 4 * q);
                 f[4 * q] = fv.x, f[4 * q + 1] = fv.y, f[4 * q + 2] = fv.z, f[4 * q + 3] = fv.w;
@@ -187,51 +216,80 @@ __global__ void __launch_bounds__(kScanThreads) k_lattice_scan(Lattice L, Partit
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < kScanItems; ++k)
+            for (int k = 0; k < ITEMS; ++k)
                 if (base + k < size) {
                     f[k] = B.lat_flag[base + k];
                     d[k] = B.dcount[base + k];
                 }
         }
     }
-    uint64_t sp = 0;
-    uint32_t sgb = 0, sgx = 0;  // grid blocks, extra parts
+    // scene of the tile's first entry: each round, the wave's lanes probe 64 evenly spaced scenes
+    int scene = 0;
+    if (L.nscenes > 1 && need) {
+        const int64_t first = (int64_t)tile * (kScanThreads * ITEMS);
+        for (int cnt = L.nscenes; cnt > 1;) {
+            const int stride = (cnt + 63) / 64, at = lane * stride;
+            const uint64_t below = __ballot(at < cnt && (int64_t)L.scenes[scene + min(at, cnt - 1)].lat_off <= first);
+            const int k = (__popcll(below) - 1) * stride;  // lane 0's scene begins at or before the entry
+            scene += k;
+            cnt = min(stride, cnt - k);
+        }
+    }
+    uint32_t sd = 0, sb = 0, sx = 0;  // particles; blocks, grid blocks << 16 (at most 4096 each); extra parts
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        sp += ((uint64_t)d[k] << kPBlkBits) | (uint64_t)(f[k] & 1u);
-        sgb += (f[k] >> 1) & 1u;
-        sgx += extra_parts(d[k], L.part_shift);  // 0 for entries without particles
+    for (int k = 0; k < ITEMS; ++k) {
+        sd += d[k];
+        sb += (f[k] & 1u) | (((f[k] >> 1) & 1u) << 16);
+        sx += extra_parts(d[k], L.part_shift);  // 0 for entries without particles
     }
-    const uint64_t sg = ((uint64_t)sgx << 32) | sgb;
-    uint64_t totp = 0, totg = 0, ep = 0, eg = 0;
+    uint32_t incl[3] = {sd, sb, sx}, tot[3] = {0u, 0u, 0u};
     if (need) {
-        ep = block_excl_scan_u64(sp, s_wave, &totp);
-        eg = block_excl_scan_u64(sg, s_wave, &totg);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            incl[q] = wave_scan_u32(incl[q]);
+            if (lane == 63) s_sum[q][w] = incl[q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int k = 0; k < NWAVE; ++k) {
+                const uint32_t x = s_sum[q][k];
+                tot[q] += x;
+                incl[q] += k < w ? x : 0u;
+            }
     }
+    const uint64_t totp = ((uint64_t)tot[0] << kPBlkBits) | (tot[1] & 0xffffu);
+    const uint64_t totg = ((uint64_t)tot[2] << 32) | (tot[1] >> 16);
     // the two chains look back concurrently, one wave each
-    __shared__ uint64_t s_pref[2];
-    if (threadIdx.x < 64) {
+    if (w == 0) {
         const uint64_t x = lookback_wave(B.scan_p, tile, totp);
-        if (threadIdx.x == 0) s_pref[0] = x;
-    } else if (threadIdx.x < 128) {
+        if (lane == 0) s_pref[0] = x;
+    } else if (w == 1) {
         const uint64_t x = lookback_wave(B.scan_g, tile, totg);
-        if (threadIdx.x == 64) s_pref[1] = x;
+        if (lane == 0) s_pref[1] = x;
     }
     __syncthreads();
     const uint64_t tp = s_pref[0], tg = s_pref[1];
     if (need) {
-        uint64_t rp = tp + ep;
-        uint32_t rg = (uint32_t)(tg + eg), rx = (uint32_t)((tg + eg) >> 32);
-        // scene of this thread's first entry; later entries advance from it
-        int scene = base < size ? scene_of(L, base) : 0;
-        int32_t op[kScanItems], og[kScanItems];
-        uint32_t xf[kScanItems / 4] = {0u, 0u, 0u, 0u};  // extra-part flags, one byte per entry
+        uint64_t rp = tp + (((uint64_t)(incl[0] - sd) << kPBlkBits) | ((incl[1] - sb) & 0xffffu));
+        uint32_t rg = (uint32_t)tg + ((incl[1] - sb) >> 16), rx = (uint32_t)(tg >> 32) + (incl[2] - sx);
+        const int64_t never = (int64_t)1 << 40;
+        int64_t next = scene + 1 < L.nscenes ? (int64_t)L.scenes[scene + 1].lat_off : never;  // the next scene's first
+        int32_t op[ITEMS], og[ITEMS];
+        uint32_t xf[ITEMS / 4] = {};  // extra-part flags, one byte per entry
+        uint32_t any = 0u;
 #pragma unroll
-        for (int k = 0; k < kScanItems; ++k) {
+        for (int k = 0; k < ITEMS; ++k) any |= f[k];
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
             const int64_t i = base + k;
             op[k] = og[k] = -1;
-            if (i >= size) continue;
-            while (scene + 1 < L.nscenes && L.scenes[scene + 1].lat_off <= i) ++scene;
+            if (any == 0u) continue;  // d is 0 wherever f is
+            while (i >= next) {
+                ++scene;
+                next = scene + 1 < L.nscenes ? (int64_t)L.scenes[scene + 1].lat_off : never;
+            }
             const uint32_t extra = extra_parts(d[k], L.part_shift);
             if (f[k] & 1u) {
                 const uint32_t pidx = (uint32_t)(rp & kBlkMask), first = (uint32_t)(rp >> kPBlkBits);
@@ -258,12 +316,12 @@ __global__ void __launch_bounds__(kScanThreads) k_lattice_scan(Lattice L, Partit
         }
         if (full) {
 #pragma unroll
-            for (int q = 0; q < kScanItems / 4; ++q) {
+            for (int q = 0; q < ITEMS / 4; ++q) {
+                *reinterpret_cast<uint32_t *>(Pn.lat_xf + base + 4 * q) = xf[q];
                 *reinterpret_cast<int4 *>(Pn.lat_pid + base + 4 * q) =
                     make_int4(op[4 * q], op[4 * q + 1], op[4 * q + 2], op[4 * q + 3]);
                 *reinterpret_cast<int4 *>(Pn.lat_gid + base + 4 * q) =
                     make_int4(og[4 * q], og[4 * q + 1], og[4 * q + 2], og[4 * q + 3]);
-                if (q == 0) *reinterpret_cast<uint4 *>(Pn.lat_xf + base) = make_uint4(xf[0], xf[1], xf[2], xf[3]);
                 if (f[4 * q] | f[4 * q + 1] | f[4 * q + 2] | f[4 * q + 3]) {
                     *reinterpret_cast<uint4 *>(B.lat_flag + base + 4 * q) = make_uint4(0u, 0u, 0u, 0u);
                     *reinterpret_cast<uint4 *>(B.dcount + base + 4 * q) = make_uint4(0u, 0u, 0u, 0u);
@@ -271,7 +329,7 @@ __global__ void __launch_bounds__(kScanThreads) k_lattice_scan(Lattice L, Partit
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < kScanItems; ++k)
+            for (int k = 0; k < ITEMS; ++k)
                 if (base + k < size) {
                     Pn.lat_pid[base + k] = op[k];
                     Pn.lat_gid[base + k] = og[k];
@@ -280,7 +338,7 @@ __global__ void __launch_bounds__(kScanThreads) k_lattice_scan(Lattice L, Partit
                     B.dcount[base + k] = 0u;
                 }
         }
-        if (threadIdx.x == 0) {
+        if (!SMALL && threadIdx.x == 0) {
             Pn.tile_used[tile] = (totp | totg) != 0u ? 1u : 0u;
             B.tile_mark[tile] = 0u;
         }
@@ -298,7 +356,6 @@ __global__ void __launch_bounds__(kScanThreads) k_lattice_scan(Lattice L, Partit
             B.host_counts[2] = (uint32_t)(ag >> 32);
         }
     }
-    if (threadIdx.x == 0 && *B.scan_p.stall_flag) atomicOr(&st->scan_stall, 1u);
 }
 
 __global__ void __launch_bounds__(kThreads) k_gather_state(State src, int64_t src_cap, State dst, int64_t dst_cap,
@@ -308,17 +365,6 @@ __global__ void __launch_bounds__(kThreads) k_gather_state(State src, int64_t sr
 #pragma unroll
         for (int c = 0; c < kTileCh; ++c) chan(dst.ch, (uint32_t)k, c) = chan(src.ch, i, c);
     }
-}
-
-// Inclusive sum over the wave's lanes by DPP row shifts and broadcasts.
-__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return v;
 }
 
 // ------------------------------------------------------------------ P2G
@@ -3354,6 +3400,15 @@ void launch_set_steps(SceneParams *scenes, int32_t nscenes, StepArgs a, int mask
                        scenes, nscenes, a, mask);
 }
 
+void launch_lattice_scan(Lattice L, Partition Pn, Binning B, const uint32_t *prev_used, hipStream_t s) {
+    if (small_scan(L.size))
+        hipLaunchKernelGGL(k_lattice_scan<true>, dim3((unsigned)B.scan_tiles), dim3(kScanThreads), 0, s, L, Pn, B,
+                           prev_used);
+    else
+        hipLaunchKernelGGL(k_lattice_scan<false>, dim3((unsigned)B.scan_tiles), dim3(kScanThreads), 0, s, L, Pn, B,
+                           prev_used);
+}
+
 void launch_partition_from_keys(const uint32_t *skeys, int64_t n, Lattice L, Partition P, Binning B, State sorted,
                                 const DevMaterial *mats, DevStatus *st, hipStream_t s) {
     // lat_flag and dcount are zero here: every scan clears the entries it was given to read
@@ -3362,8 +3417,7 @@ void launch_partition_from_keys(const uint32_t *skeys, int64_t n, Lattice L, Par
         hipLaunchKernelGGL(k_mark_blocks, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, skeys, n, L,
                            (const float *)sorted.ch, mats, B.lat_flag, B.dcount);
     // the scan forms the block starts from the counts k_mark_blocks left in dcount
-    hipLaunchKernelGGL(k_lattice_scan, dim3((unsigned)B.scan_tiles), dim3(kScanThreads), 0, s, L, P, B,
-                       (const uint32_t *)P.tile_used, st);
+    launch_lattice_scan(L, P, B, (const uint32_t *)P.tile_used, s);
 }
 
 void launch_gather_state(State src, int64_t src_cap, State dst, int64_t dst_cap, const uint32_t *perm, int64_t n,
@@ -3551,13 +3605,6 @@ void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float
     }
     hipLaunchKernelGGL(k_permute_channels, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, layout, nch, n, src, dst,
                        order, staging ? (const uint32_t *)staged : nullptr);
-}
-
-void launch_lattice_scan(Lattice L, Partition Pn, Binning B, const uint32_t *prev_used, int64_t n, DevStatus *st,
-                         hipStream_t s) {
-    (void)n;
-    hipLaunchKernelGGL(k_lattice_scan, dim3((unsigned)B.scan_tiles), dim3(kScanThreads), 0, s, L, Pn, B, prev_used,
-                       st);
 }
 
 void launch_g2p_update(bool scatter, State A, State Bst, Partition P, Partition Pn, Lattice L, const float *grid,

@@ -424,7 +424,8 @@ zmpm_ctx *create_context(const zmpm_scene *scenes, int32_t nscenes, int64_t capa
         B.code = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         B.mvlist = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->arr = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
-        B.scan_tiles = (L + kScanTile - 1) / kScanTile;
+        const int64_t scan_tile = small_scan(L) ? kSmallScanTile : kScanTile;
+        B.scan_tiles = (L + scan_tile - 1) / scan_tile;
         B.tile_mark = (uint32_t *)c->alloc(sizeof(uint32_t) * B.scan_tiles);
         int64_t nbmax = 0;
         for (const SceneParams &q : sp) nbmax = std::max<int64_t>(nbmax, q.nb);
@@ -435,8 +436,6 @@ zmpm_ctx *create_context(const zmpm_scene *scenes, int32_t nscenes, int64_t capa
         B.scan_g.status = (uint64_t *)c->alloc(sizeof(uint64_t) * B.scan_tiles);
         B.scan_p.tile_ctr = (uint32_t *)c->alloc(sizeof(uint32_t) * 4);
         B.scan_g.tile_ctr = B.scan_p.tile_ctr;
-        B.scan_p.stall_flag = B.scan_p.tile_ctr + 1;
-        B.scan_g.stall_flag = B.scan_p.tile_ctr + 1;
         HIP_CHECK(hipMemset(B.lat_flag, 0, sizeof(uint32_t) * L));
         HIP_CHECK(hipMemset(B.dcount, 0, sizeof(uint32_t) * L));
         HIP_CHECK(hipMemset(B.scan_p.tile_ctr, 0, sizeof(uint32_t) * 4));
@@ -454,6 +453,7 @@ zmpm_ctx *create_context(const zmpm_scene *scenes, int32_t nscenes, int64_t capa
         c->grid = (float *)c->alloc(sizeof(float) * 256 * c->grid_blocks);
         c->status = (DevStatus *)c->alloc(sizeof(DevStatus));
         HIP_CHECK(hipMemset(c->status, 0, sizeof(DevStatus)));
+        B.scan_p.stall_flag = B.scan_g.stall_flag = &c->status->scan_stall;
         c->mats = (DevMaterial *)c->alloc(sizeof(DevMaterial) * kMaxMaterials);
         HIP_CHECK(hipDeviceSynchronize());
     } catch (...) {
@@ -1180,7 +1180,7 @@ void substep_fused(zmpm_ctx *ctx, hipEvent_t *ev, int grow, bool last) {
     launch_g2p_move(A, P, ctx->L, ctx->grid, ctx->gvmax, ctx->bin, ctx->status, npb, s, ctx->wg_move(), nullptr, false,
                     true);
     if (ev) HIP_CHECK(hipEventRecord(ev[4], s));
-    launch_lattice_scan(ctx->L, Pn, ctx->bin, P.tile_used, ctx->n, ctx->status, s);
+    launch_lattice_scan(ctx->L, Pn, ctx->bin, P.tile_used, s);
     ctx->psize[ctx->pcur ^ 1] = ctx->L.part_shift;
     if (ev) HIP_CHECK(hipEventRecord(ev[5], s));
     // the new partition's blocks: at most the old count plus what the lattice scan adds, as G2P update sizes it
@@ -1262,7 +1262,7 @@ void substep_once(zmpm_ctx *ctx, hipEvent_t *ev, int grow = 0, bool last = true)
                     nonaffine);
     if (ev) HIP_CHECK(hipEventRecord(ev[4], s));
     // the next partition: particle blocks, their first particles, grid blocks
-    launch_lattice_scan(ctx->L, Pn, ctx->bin, P.tile_used, ctx->n, ctx->status, s);
+    launch_lattice_scan(ctx->L, Pn, ctx->bin, P.tile_used, s);
     ctx->psize[ctx->pcur ^ 1] = ctx->L.part_shift;
     if (ev) HIP_CHECK(hipEventRecord(ev[5], s));
     // G2P pass 2: full update, written straight into the next stable block order

@@ -290,8 +290,7 @@ void launch_g2p2g(State A, State B, Partition P, Partition Pn, Lattice L, const 
                   bool general, int64_t n, int64_t max_blocks, hipStream_t s);
 // Lattice scan: the new partition from the destination marks and particle counts.
 // prev_used: tile_used of the partition the particles move from
-void launch_lattice_scan(Lattice L, Partition Pn, Binning B, const uint32_t *prev_used, int64_t n, DevStatus *st,
-                         hipStream_t s);
+void launch_lattice_scan(Lattice L, Partition Pn, Binning B, const uint32_t *prev_used, hipStream_t s);
 // G2P update: in place (scatter == false), or written into the next stable block order.
 // aux: kAux* channels the scatter carries; nonaffine: the FLIP transfer (velocity
 // gradient from the weight gradients, C kept).
