@@ -37,6 +37,20 @@ __device__ __forceinline__ void bspline_dw(float f, float dw[3]) {
     dw[2] = f - 0.5f;
 }
 
+// a[k] of a register array for a k known only at run time (an index would put the array into scratch)
+__device__ __forceinline__ float pick3(const float a[3], int k) { return k == 0 ? a[0] : (k == 1 ? a[1] : a[2]); }
+
+// What an adjoint gather needs of a particle first.
+struct AdjParticle {
+    float x[3];
+    uint32_t mw, pid;
+};
+__device__ __forceinline__ AdjParticle adj_particle(const State &A, uint32_t i) {
+    return {{chan(A.ch, i, kChX), chan(A.ch, i, kChX + 1), chan(A.ch, i, kChX + 2)},
+            chan_u(A.ch, i, kChMat),
+            chan_u(A.ch, i, kChPid)};
+}
+
 // Per grid block, dL/dm and dL/dmv of the 6^3 stencil region as float4 (m, mv).
 __device__ __forceinline__ void stage_block_grid4(float4 *s_g, const float *grid, const int32_t *lat_gid, int64_t l,
                                                   int64_t nb, int64_t nb2) {
@@ -64,20 +78,22 @@ __global__ void __launch_bounds__(kAdjThreads) k_g2p_adjoint(State A, Partition 
     const int64_t n = adj.n;
     const uint32_t chunk = blockIdx.x % kAdjChunks;
     for (uint32_t b = blockIdx.x / kAdjChunks; b < nblocks; b += gridDim.x / kAdjChunks) {
+        const uint32_t ps = P.pblk_start[b], pe = P.pblk_start[b + 1];
         const int64_t l = P.pblk_lat[b];
+        if (ps + chunk * kAdjThreads >= pe) continue;
         const SceneParams sc = scene_params(L, L.nscenes == 1 ? 0u : P.pblk_scene[b]);
         const int64_t nb = sc.nb, nb2 = nb * nb;
         int lb[3];
         lattice_coords(sc, l, lb[0], lb[1], lb[2]);
         const int bc[3] = {(lb[0] + L.origin) * 4, (lb[1] + L.origin) * 4, (lb[2] + L.origin) * 4};
+        // the first particle is read before the staging, whose loads it does not wait for
+        uint32_t i = ps + chunk * kAdjThreads + t;
+        AdjParticle pt = adj_particle(A, min(i, pe - 1u));
         stage_block_velocity<kAdjThreads>(s_v, gridv, P.lat_gid, l, nb, nb2);
         __syncthreads();
-        const uint32_t ps = P.pblk_start[b], pe = P.pblk_start[b + 1];
-        for (uint32_t i = ps + chunk * kAdjThreads + t; i < pe; i += kAdjChunks * kAdjThreads) {
-            float xp[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) xp[k] = chan(A.ch, i, kChX + k);
-            const uint32_t mw = chan_u(A.ch, i, kChMat), pid = chan_u(A.ch, i, kChPid);
+        for (; i < pe; i += kAdjChunks * kAdjThreads, pt = adj_particle(A, min(i, pe - 1u))) {
+            const float *xp = pt.x;
+            const uint32_t mw = pt.mw, pid = pt.pid;
             const bool fcr = (mw & kMatF) != 0u;
             Arena ar;
             make_arena(xp, sc.dxinv, ar);
@@ -134,26 +150,39 @@ __global__ void __launch_bounds__(kAdjThreads) k_g2p_adjoint(State A, Partition 
             float dw[3][3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) bspline_dw(ar.f[k], dw[k]);
-            float gx[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-            for (int ox = 0; ox < 3; ++ox)
+            // line by line along z: s = v_i . t with t = a + B d advanced by B's last column, then the sums
+            // of s w_z and s w'_z into the three directions
+            float gx[3] = {0.0f, 0.0f, 0.0f}, tz[3];
 #pragma unroll
-                for (int oy = 0; oy < 3; ++oy)
+            for (int r = 0; r < 3; ++r) tz[r] = Bq[r][2] * sc.dx;
+#pragma unroll 1
+            for (int ox = 0; ox < 3; ++ox) {
+                const float wx = pick3(ar.w[0], ox), dwx = pick3(dw[0], ox), d0 = ((float)ox - ar.f[0]) * sc.dx;
+                float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;  // sums over y of w_y S, w'_y S, w_y S'
+#pragma unroll
+                for (int oy = 0; oy < 3; ++oy) {
+                    const float d1 = ((float)oy - ar.f[1]) * sc.dx, d2 = -ar.f[2] * sc.dx;
+                    float t3[3], S = 0.0f, Sd = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 3; ++r)
+                        t3[r] = fmaf(Bq[r][2], d2, fmaf(Bq[r][1], d1, fmaf(Bq[r][0], d0, vb[r])));
 #pragma unroll
                     for (int oz = 0; oz < 3; ++oz) {
                         const float4 v4 = s_v[((lc[0] + ox) * kTileSide + (lc[1] + oy)) * kTileSide + lc[2] + oz];
-                        const float d[3] = {((float)ox - ar.f[0]) * sc.dx, ((float)oy - ar.f[1]) * sc.dx,
-                                            ((float)oz - ar.f[2]) * sc.dx};
-                        const float vi[3] = {v4.x, v4.y, v4.z};
-                        float s = 0.0f;
+                        const float q = fmaf(v4.x, t3[0], fmaf(v4.y, t3[1], v4.z * t3[2]));
+                        S = fmaf(q, ar.w[2][oz], S);
+                        Sd = fmaf(q, dw[2][oz], Sd);
 #pragma unroll
-                        for (int r = 0; r < 3; ++r)
-                            s += vi[r] * (vb[r] + Bq[r][0] * d[0] + Bq[r][1] * d[1] + Bq[r][2] * d[2]);
-                        const float wx = ar.w[0][ox], wy = ar.w[1][oy], wz = ar.w[2][oz];
-                        gx[0] += s * dw[0][ox] * wy * wz;
-                        gx[1] += s * wx * dw[1][oy] * wz;
-                        gx[2] += s * wx * wy * dw[2][oz];
+                        for (int r = 0; r < 3; ++r) t3[r] += tz[r];
                     }
+                    s0 = fmaf(S, ar.w[1][oy], s0);
+                    s1 = fmaf(S, dw[1][oy], s1);
+                    s2 = fmaf(Sd, ar.w[1][oy], s2);
+                }
+                gx[0] = fmaf(s0, dwx, gx[0]);
+                gx[1] = fmaf(s1, wx, gx[1]);
+                gx[2] = fmaf(s2, wx, gx[2]);
+            }
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 const float bt = Bq[0][k] * vel[0] + Bq[1][k] * vel[1] + Bq[2][k] * vel[2];
@@ -217,25 +246,26 @@ __global__ void __launch_bounds__(kAdjThreads) k_p2g_adjoint(State A, Partition 
     const int64_t n = adj.n;
     const uint32_t chunk = blockIdx.x % kAdjChunks;
     for (uint32_t b = blockIdx.x / kAdjChunks; b < nblocks; b += gridDim.x / kAdjChunks) {
+        const uint32_t ps = P.pblk_start[b], pe = P.pblk_start[b + 1];
         const int64_t l = P.pblk_lat[b];
+        if (ps + chunk * kAdjThreads >= pe) continue;
         const SceneParams sc = scene_params(L, L.nscenes == 1 ? 0u : P.pblk_scene[b]);
         const int64_t nb = sc.nb, nb2 = nb * nb;
         int lb[3];
         lattice_coords(sc, l, lb[0], lb[1], lb[2]);
         const int bc[3] = {(lb[0] + L.origin) * 4, (lb[1] + L.origin) * 4, (lb[2] + L.origin) * 4};
+        uint32_t i = ps + chunk * kAdjThreads + t;
+        AdjParticle pt = adj_particle(A, min(i, pe - 1u));
         stage_block_grid4(s_g, gbar, P.lat_gid, l, nb, nb2);
         __syncthreads();
-        const uint32_t ps = P.pblk_start[b], pe = P.pblk_start[b + 1];
-        for (uint32_t i = ps + chunk * kAdjThreads + t; i < pe; i += kAdjChunks * kAdjThreads) {
-            float xp[3], vp[3], Cp[3][3];
+        for (; i < pe; i += kAdjChunks * kAdjThreads, pt = adj_particle(A, min(i, pe - 1u))) {
+            float vp[3], Cp[3][3];
+            const float *xp = pt.x;
+            const uint32_t mw = pt.mw, pid = pt.pid;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                xp[k] = chan(A.ch, i, kChX + k);
-                vp[k] = chan(A.ch, i, kChV + k);
-            }
+            for (int k = 0; k < 3; ++k) vp[k] = chan(A.ch, i, kChV + k);
 #pragma unroll
             for (int q = 0; q < 9; ++q) Cp[q / 3][q % 3] = chan(A.ch, i, kChC + q);
-            const uint32_t mw = chan_u(A.ch, i, kChMat), pid = chan_u(A.ch, i, kChPid);
             const DevMaterial mt = mats[mw & kMatIndexMask];
             const bool fcr = mt.model == ZMPM_MODEL_FCR;
             // the particle's own m, vol when it carries them (Transfer.cu:857-858)
@@ -272,33 +302,63 @@ __global__ void __launch_bounds__(kAdjThreads) k_p2g_adjoint(State A, Partition 
             float dw[3][3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) bspline_dw(ar.f[k], dw[k]);
-            float G0[3] = {0.0f, 0.0f, 0.0f}, Bb[3][3] = {{0.0f}}, gx[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-            for (int ox = 0; ox < 3; ++ox)
+            // line by line along z, as in the G2P adjoint: per node the momentum m v + B d the particle
+            // sends there (advanced by B's last column) and q = g_m m + g_mv . momentum; per line the sums
+            // of w_z g_mv, w_z d_z g_mv, q w_z and q w'_z
+            float G0[3] = {0.0f, 0.0f, 0.0f}, Bb[3][3] = {{0.0f}}, gx[3] = {0.0f, 0.0f, 0.0f}, tz[3];
 #pragma unroll
-                for (int oy = 0; oy < 3; ++oy)
+            for (int r = 0; r < 3; ++r) tz[r] = Bm[r][2] * sc.dx;
+#pragma unroll 1
+            for (int ox = 0; ox < 3; ++ox) {
+                const float wx = pick3(ar.w[0], ox), dwx = pick3(dw[0], ox), d0 = ((float)ox - ar.f[0]) * sc.dx;
+                float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
+                float p0[3] = {0.0f, 0.0f, 0.0f}, py[3] = {0.0f, 0.0f, 0.0f}, pz[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int oy = 0; oy < 3; ++oy) {
+                    const float d1 = ((float)oy - ar.f[1]) * sc.dx, wy = ar.w[1][oy];
+                    float t3[3], l0[3] = {0.0f, 0.0f, 0.0f}, lz[3] = {0.0f, 0.0f, 0.0f}, S = 0.0f, Sd = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 3; ++r)
+                        t3[r] = fmaf(Bm[r][2], -ar.f[2] * sc.dx, fmaf(Bm[r][1], d1, fmaf(Bm[r][0], d0, m * vp[r])));
 #pragma unroll
                     for (int oz = 0; oz < 3; ++oz) {
                         const float4 g4 = s_g[((lc[0] + ox) * kTileSide + (lc[1] + oy)) * kTileSide + lc[2] + oz];
-                        const float d[3] = {((float)ox - ar.f[0]) * sc.dx, ((float)oy - ar.f[1]) * sc.dx,
-                                            ((float)oz - ar.f[2]) * sc.dx};
-                        const float wx = ar.w[0][ox], wy = ar.w[1][oy], wz = ar.w[2][oz];
-                        const float W = wx * wy * wz;
                         const float mvb[3] = {g4.y, g4.z, g4.w};
-                        // mass and momentum the particle sends to node i (for the weight gradient)
+                        const float wz = ar.w[2][oz], wdz = wz * (((float)oz - ar.f[2]) * sc.dx);
                         float q = g4.x * m;
 #pragma unroll
                         for (int r = 0; r < 3; ++r) {
-                            const float mom = m * vp[r] + Bm[r][0] * d[0] + Bm[r][1] * d[1] + Bm[r][2] * d[2];
-                            q += mvb[r] * mom;
-                            G0[r] += W * mvb[r];
-#pragma unroll
-                            for (int c = 0; c < 3; ++c) Bb[r][c] += W * mvb[r] * d[c];
+                            q = fmaf(mvb[r], t3[r], q);
+                            l0[r] = fmaf(wz, mvb[r], l0[r]);
+                            lz[r] = fmaf(wdz, mvb[r], lz[r]);
+                            t3[r] += tz[r];
                         }
-                        gx[0] += q * dw[0][ox] * wy * wz;
-                        gx[1] += q * wx * dw[1][oy] * wz;
-                        gx[2] += q * wx * wy * dw[2][oz];
+                        S = fmaf(q, wz, S);
+                        Sd = fmaf(q, dw[2][oz], Sd);
                     }
+                    const float wdy = wy * d1;
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) {
+                        p0[r] = fmaf(wy, l0[r], p0[r]);
+                        py[r] = fmaf(wdy, l0[r], py[r]);
+                        pz[r] = fmaf(wy, lz[r], pz[r]);
+                    }
+                    s0 = fmaf(S, wy, s0);
+                    s1 = fmaf(S, dw[1][oy], s1);
+                    s2 = fmaf(Sd, wy, s2);
+                }
+                const float wd0 = wx * d0;
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    G0[r] = fmaf(wx, p0[r], G0[r]);
+                    Bb[r][0] = fmaf(wd0, p0[r], Bb[r][0]);
+                    Bb[r][1] = fmaf(wx, py[r], Bb[r][1]);
+                    Bb[r][2] = fmaf(wx, pz[r], Bb[r][2]);
+                }
+                gx[0] = fmaf(s0, dwx, gx[0]);
+                gx[1] = fmaf(s1, wx, gx[1]);
+                gx[2] = fmaf(s2, wx, gx[2]);
+            }
             // x: weight gradient, and d_i = x_i - x contributes -B^T G0
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
