@@ -74,31 +74,13 @@ __device__ __forceinline__ uint32_t particle_key(const float *x, int64_t stride,
     return position_key(xp, scene_params(L, (uint32_t)scene), L.origin, L.key_shift, bad);
 }
 
-// check: also flag (bin_mismatch) a state whose blocks are out of order, which a
-// state assumed to be in stable block order must not be.
 __global__ void __launch_bounds__(kThreads) k_bin_keys(const float *x, int64_t stride, int64_t n,
                                                        const DevMaterial *mats, Lattice L, uint32_t *keys,
-                                                       DevStatus *st, int check) {
-    bool bad = false, unsorted = false;
-    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
-        const uint32_t key = particle_key(x, stride, i, mats, L, bad);
-        keys[i] = key;
-        if (check && i > 0)
-            unsorted |= (particle_key(x, stride, i - 1, mats, L, bad) >> L.key_shift) > (key >> L.key_shift);
-    }
+                                                       DevStatus *st) {
+    bool bad = false;
+    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
+        keys[i] = particle_key(x, stride, i, mats, L, bad);
     if (bad) atomicOr(&st->domain_error, 1u);
-    if (unsorted) atomicOr(&st->bin_mismatch, 1u);
-}
-
-// Resets the lattice scan's look-back state; force: make the scan visit every tile.
-__global__ void __launch_bounds__(kThreads) k_scan_reset(Binning B, uint32_t force) {
-    for (int64_t k = blockIdx.x * (int64_t)kThreads + threadIdx.x; k < B.scan_tiles;
-         k += (int64_t)gridDim.x * kThreads) {
-        B.scan_p.status[k] = 0ull;
-        B.scan_g.status[k] = 0ull;
-        B.tile_mark[k] = force;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *B.scan_p.tile_ctr = 0u;
 }
 
 // ------------------------------------------------------------------ partition
@@ -110,16 +92,33 @@ __global__ void __launch_bounds__(kThreads) k_scan_reset(Binning B, uint32_t for
 // Each block's particle count goes to dcount (one atomic per run of one block within a
 // wave), from which the lattice scan forms the block starts and parts, as it does for the
 // counts of the move pass.
+// It also resets the scan's look-back state and makes the scan visit every tile (tile_mark).
+// skeys null: the keys of a state that is assumed to be in stable block order (a saved one), made
+// here; blocks out of order are flagged (bin_mismatch).  (A re-bin of 131,072 saved particles took
+// three launches, keys, reset and marks, 4.6 + 4.2 + 4.4 us; this one 4.7.)
 __global__ void __launch_bounds__(kThreads) k_mark_blocks(const uint32_t *skeys, int64_t n, Lattice L,
-                                                          const float *ch, const DevMaterial *mats,
-                                                          uint32_t *lat_flag, uint32_t *dcount) {
+                                                          const float *ch, const DevMaterial *mats, Binning B,
+                                                          DevStatus *st) {
     const int lane = threadIdx.x & 63;
-    for (int64_t k0 = blockIdx.x * (int64_t)kThreads; k0 < n; k0 += (int64_t)gridDim.x * kThreads) {  // uniform
+    uint32_t *lat_flag = B.lat_flag, *dcount = B.dcount;
+    const int64_t gtid = blockIdx.x * (int64_t)kThreads + threadIdx.x, gsz = (int64_t)gridDim.x * kThreads;
+    for (int64_t k = gtid; k < B.scan_tiles; k += gsz) {
+        B.scan_p.status[k] = 0ull;
+        B.scan_g.status[k] = 0ull;
+        B.tile_mark[k] = 1u;
+    }
+    if (gtid == 0) *B.scan_p.tile_ctr = 0u;
+    bool bad = false, unsorted = false;
+    for (int64_t k0 = blockIdx.x * (int64_t)kThreads; k0 < n; k0 += gsz) {  // uniform
         const int64_t k = k0 + threadIdx.x;
         const bool valid = k < n;
-        const uint32_t blk = valid ? skeys[k] >> L.key_shift : 0xffffffffu;
-        const uint32_t prev = __shfl_up(blk, 1, 64);
-        if (valid && (k == 0 || (skeys[k - 1] >> L.key_shift) != blk)) {
+        uint32_t blk = 0xffffffffu;
+        if (valid) blk = (skeys ? skeys[k] : particle_key(ch, -1, k, mats, L, bad)) >> L.key_shift;
+        uint32_t prev = __shfl_up(blk, 1, 64);
+        if (valid && lane == 0 && k > 0)
+            prev = (skeys ? skeys[k - 1] : particle_key(ch, -1, k - 1, mats, L, bad)) >> L.key_shift;
+        if (valid && k > 0) unsorted |= prev > blk;
+        if (valid && (k == 0 || prev != blk)) {
             const int64_t nb = L.scenes[mats[chan_u(ch, (uint32_t)k, kChMat) & kMatIndexMask].scene].nb;
             const int64_t nb2 = nb * nb;
 #pragma unroll
@@ -137,6 +136,8 @@ __global__ void __launch_bounds__(kThreads) k_mark_blocks(const uint32_t *skeys,
             atomicAdd(&dcount[blk], (uint32_t)(end - lane));
         }
     }
+    if (bad) atomicOr(&st->domain_error, 1u);
+    if (unsorted) atomicOr(&st->bin_mismatch, 1u);
 }
 
 // Inclusive sum over the wave's lanes by DPP row shifts and broadcasts.
@@ -2799,31 +2800,38 @@ __device__ __forceinline__ void rec_get(float *s, float (&v)[kRec], const float 
 }
 
 // *staged = the order (perm, or the caller indices of the resident particles) is far from the
-// memory's: 64 runs of 64 entries, evenly over the n >= 64, hold more than kLocalLines different
-// lines of 32 entries each on average (neighbours compared, so a line met again counts again).
-// 2,000,000 particles shuffled within windows of 1, 64, 256, 4,096 and all entries hold 7, 10, 25, 47
-// and 64 lines: an export takes 184, 218, 369, 638 and 972 us directly, 205 through records; an
+// memory's: 64 runs of 64 entries, evenly over the n >= 64, hold more than `lines` different
+// lines of 32 entries each on average (neighbours compared, so a line met again counts again); for an
+// export 10, and 16 for J-fluid particles, which move 17 channels in place of 25.
+// 2,000,000 solid particles shuffled within windows of 1, 64, 256, 4,096 and all entries hold 7, 10,
+// 25, 47 and 64 lines: an export takes 184, 218, 369, 638 and 972 us directly, 205 through records; an
 // import with its sort 319, 347, 417, 522 and 1,057, against 385.  At 600,000 the export: 63, 82, 116,
-// 159 and 203, against 71.
-constexpr uint32_t kLocalLines = 12;
-__global__ void __launch_bounds__(1024) k_order_sample(const uint32_t *perm, const float *ch, int64_t n,
-                                                       uint32_t *staged) {
-    __shared__ uint32_t s_lines[16];
+// 159 and 203, against 71.  The dam of 4.2 million, 93 % fluid, 12 to 16 lines: 250 directly, 353.
+__global__ void __launch_bounds__(1024) k_order_sample(const uint32_t *perm, uint32_t lines, const float *ch,
+                                                       int64_t n, uint32_t *staged) {
+    __shared__ uint32_t s_lines[16], s_fluid[16];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t lines = 0;
+    uint32_t found = 0, fluid = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int64_t k = (n - 64) * (4 * w + q) / 63 + lane;
         const uint32_t line = (perm ? perm[k] : chan_u(ch, (uint32_t)k, kChPid)) >> 5;
         const uint32_t prev = (uint32_t)__shfl_up((int)line, 1, 64);
-        lines += (uint32_t)__popcll(__ballot(lane == 0 || line != prev));
+        found += (uint32_t)__popcll(__ballot(lane == 0 || line != prev));
+        if (!perm) fluid += (uint32_t)__popcll(__ballot((chan_u(ch, (uint32_t)k, kChMat) & kMatF) == 0u));
     }
-    if (lane == 0) s_lines[w] = lines;
+    if (lane == 0) {
+        s_lines[w] = found;
+        s_fluid[w] = fluid;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t total = 0;
-        for (int q = 0; q < 16; ++q) total += s_lines[q];
-        *staged = total > 64u * kLocalLines ? 1u : 0u;
+        uint32_t total = 0, nf = 0;
+        for (int q = 0; q < 16; ++q) {
+            total += s_lines[q];
+            nf += s_fluid[q];
+        }
+        *staged = total * 64u > (perm ? lines * 4096u : 10u * 4096u + 6u * nf) ? 1u : 0u;
     }
 }
 
@@ -3388,10 +3396,9 @@ void launch_extract_pid(State A, int64_t n, uint32_t *out, hipStream_t s) {
 }
 
 void launch_bin_keys(const float *x, int64_t stride, int64_t n, const DevMaterial *mats, Lattice L, uint32_t *keys,
-                     DevStatus *st, hipStream_t s, bool check_sorted) {
+                     DevStatus *st, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_bin_keys, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, x, stride, n, mats, L, keys, st,
-                       check_sorted ? 1 : 0);
+    hipLaunchKernelGGL(k_bin_keys, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, x, stride, n, mats, L, keys, st);
 }
 
 void launch_set_steps(SceneParams *scenes, int32_t nscenes, StepArgs a, int mask, hipStream_t s) {
@@ -3412,10 +3419,8 @@ void launch_lattice_scan(Lattice L, Partition Pn, Binning B, const uint32_t *pre
 void launch_partition_from_keys(const uint32_t *skeys, int64_t n, Lattice L, Partition P, Binning B, State sorted,
                                 const DevMaterial *mats, DevStatus *st, hipStream_t s) {
     // lat_flag and dcount are zero here: every scan clears the entries it was given to read
-    hipLaunchKernelGGL(k_scan_reset, dim3(grid_for(B.scan_tiles, 1024)), dim3(kThreads), 0, s, B, 1u);
-    if (n > 0)
-        hipLaunchKernelGGL(k_mark_blocks, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, skeys, n, L,
-                           (const float *)sorted.ch, mats, B.lat_flag, B.dcount);
+    hipLaunchKernelGGL(k_mark_blocks, dim3(grid_for(std::max<int64_t>(n, 1), 8192)), dim3(kThreads), 0, s, skeys, n, L,
+                       (const float *)sorted.ch, mats, B, st);
     // the scan forms the block starts from the counts k_mark_blocks left in dcount
     launch_lattice_scan(L, P, B, (const uint32_t *)P.tile_used, s);
 }
@@ -3597,7 +3602,7 @@ void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float
     if (n <= 0) return;
     const bool staging = rec && nch <= kRec && layout != ZMPM_LAYOUT_AOS && n >= kStageMin;
     if (staging) {
-        launch_order_sample(order, State{}, n, staged, s);
+        launch_order_sample(order, kMortonLines, State{}, n, staged, s);
         hipLaunchKernelGGL(k_channels_to_rec, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, layout, nch, n, src, rec,
                            (const uint32_t *)staged);
         hipLaunchKernelGGL(k_rec_to_channels, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, layout, nch, n,
@@ -3654,8 +3659,8 @@ void launch_import(State dst, const void *view, int64_t off, const DevMaterial *
     hipLaunchKernelGGL(k_import, dim3(grid_for(v.n, 8192)), dim3(kThreads), 0, s, dst, v, off, mats, nmat, st);
 }
 
-void launch_order_sample(const uint32_t *perm, State A, int64_t n, uint32_t *staged, hipStream_t s) {
-    hipLaunchKernelGGL(k_order_sample, dim3(1), dim3(1024), 0, s, perm, (const float *)A.ch, n, staged);
+void launch_order_sample(const uint32_t *perm, uint32_t lines, State A, int64_t n, uint32_t *staged, hipStream_t s) {
+    hipLaunchKernelGGL(k_order_sample, dim3(1), dim3(1024), 0, s, perm, lines, (const float *)A.ch, n, staged);
 }
 
 void launch_view_keys(const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, Lattice L, uint32_t *keys,

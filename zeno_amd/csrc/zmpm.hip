@@ -278,7 +278,7 @@ void import_sorted(zmpm_ctx *c, const zmpm_particles *views, int32_t nviews, boo
     sort_by_block(c);
     float *rec = records ? c->st[c->cur].ch : nullptr;
     uint32_t *staged = records && nviews == 1 ? c->staged : nullptr;
-    if (staged) launch_order_sample(c->perm, State{}, c->n, staged, s);
+    if (staged) launch_order_sample(c->perm, kImportLines, State{}, c->n, staged, s);
     off = 0;
     for (int k = 0; rec && k < nviews; off += views[k++].n)
         launch_view_to_rec(&views[k], off, c->mats, c->nmat, rec, staged, s);
@@ -299,9 +299,9 @@ void full_partition(zmpm_ctx *c, uint32_t part_shift = 0, bool sorted = false) {
     State A = c->st[c->cur], B = c->st[c->cur ^ 1];
     // a saved state is already in stable block order: the sort would be the identity
     // (a state that is not is reported as a binning inconsistency at the next sync)
-    if (!sorted) launch_bin_keys(A.ch, -1, c->n, c->mats, c->L, c->keys, c->status, s, c->loaded_sorted);
+    if (!sorted && !c->loaded_sorted) launch_bin_keys(A.ch, -1, c->n, c->mats, c->L, c->keys, c->status, s);
     if (c->loaded_sorted) {
-        launch_partition_from_keys(c->keys, c->n, c->L, c->part[c->pcur], c->bin, A, c->mats, c->status, s);
+        launch_partition_from_keys(nullptr, c->n, c->L, c->part[c->pcur], c->bin, A, c->mats, c->status, s);
         c->loaded_sorted = false;
     } else {
         if (!sorted) {
@@ -693,7 +693,7 @@ void export_views(zmpm_ctx *ctx, const zmpm_particles *views, int32_t nviews) {
                 (views[k].a ? kAuxFiber : 0) | (views[k].m ? kAuxMass : 0);
     uint32_t *staged = ctx->n >= kStageMin && !(want & kAuxFiber) ? ctx->staged : nullptr;
     if (staged) {
-        launch_order_sample(nullptr, ctx->st[ctx->cur], ctx->n, staged, ctx->stream);
+        launch_order_sample(nullptr, 0, ctx->st[ctx->cur], ctx->n, staged, ctx->stream);
         launch_export_to_rec(ctx->st[ctx->cur], ctx->n, ctx->mats, ctx->aux(), want, ctx->records(), staged,
                              ctx->stream);
     }

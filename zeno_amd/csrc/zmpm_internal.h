@@ -214,13 +214,13 @@ void launch_set_steps(SceneParams *scenes, int32_t nscenes, StepArgs a, int mask
 
 // x: SoA planes x[k * stride + i], or the resident tiled state when stride < 0.
 // Scene of each particle: mats[material].scene for the resident state; scene 0 for SoA input.
-// check_sorted: status->bin_mismatch if the particles' blocks are not in nondecreasing order
 void launch_bin_keys(const float *x, int64_t stride, int64_t n, const DevMaterial *mats, Lattice L, uint32_t *keys,
-                     DevStatus *st, hipStream_t s, bool check_sorted = false);
+                     DevStatus *st, hipStream_t s);
 // out[i] = caller index of resident particle i
 void launch_extract_pid(State A, int64_t n, uint32_t *out, hipStream_t s);
 // Partition of a key array sorted by block (the full re-bin path); `sorted` is the
-// state already permuted into that order (for the per-block material flags).
+// state already permuted into that order (for the per-block material flags).  skeys null: the keys of
+// `sorted`, with status->bin_mismatch if its blocks are not in nondecreasing order.
 void launch_partition_from_keys(const uint32_t *skeys, int64_t n, Lattice L, Partition P, Binning B, State sorted,
                                 const DevMaterial *mats, DevStatus *st, hipStream_t s);
 // number of scenes a launch may address through SceneParams::lat_off lookups
@@ -327,8 +327,9 @@ void launch_view_to_rec(const void *view, int64_t off, const DevMaterial *mats, 
 void launch_import_sorted(State dst, const void *view, const float *rec, const uint32_t *perm, int64_t n,
                           const DevMaterial *mats, int32_t nmat, const uint32_t *staged, hipStream_t s);
 // *staged = whether perm (null: the resident particles' caller indices) is so far from memory order
-// that moving the particles through records is the faster way (n >= 64)
-void launch_order_sample(const uint32_t *perm, State A, int64_t n, uint32_t *staged, hipStream_t s);
+// that moving the particles through records is the faster way (n >= 64): more than `lines` lines a run
+constexpr uint32_t kImportLines = 16, kMortonLines = 12;
+void launch_order_sample(const uint32_t *perm, uint32_t lines, State A, int64_t n, uint32_t *staged, hipStream_t s);
 // aux: the kAux* channels the resident state keeps (the others are exported as their initial values);
 // the resident particles of caller index off .. off + view->n - 1 go to the view's entries 0 .. n - 1.
 // With staged, only one of launch_export and launch_export_to_rec + launch_rec_to_view does the work.
