@@ -472,7 +472,7 @@ ZMPM_API int32_t zmpm_order_by_morton_code(zmpm_ctx *ctx, int32_t layout, int32_
 
 /* zmpm_sort_keys without a context and without any device allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under HIP graph capture,
- * tight serving loops, hosts that forbid hipMalloc).  The sort's scratch is a static 9 MiB
+ * tight serving loops, hosts that forbid hipMalloc).  The sort's scratch is a static 8.5 MiB
  * device array inside libzmpm.so, held on every GPU the library runs on until the process ends,
  * which bounds n to 1,048,576 keys (ZMPM_ERR_CAPACITY above that).  Runs on the current device,
  * asynchronously on stream (0 = default stream); same results as zmpm_sort_keys (stable, bit-exact).

@@ -1736,7 +1736,7 @@ int32_t zmpm_key_bits(const zmpm_ctx *ctx) { return ctx ? ctx->key_bits : -1; }
 namespace {
 
 constexpr int64_t kNoAllocMaxKeys = (int64_t)1 << 20;
-constexpr size_t kNoAllocScratchBytes = radix_scratch_bound(kNoAllocMaxKeys);  // 9 MiB + 512 B
+constexpr size_t kNoAllocScratchBytes = radix_scratch_bound(kNoAllocMaxKeys);  // 8.5 MiB + 1 KiB
 constexpr int kNoAllocMaxDevices = 64;
 
 struct NoAllocScratch {
