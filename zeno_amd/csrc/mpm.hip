@@ -1974,19 +1974,32 @@ k_g2p_move(State A, Partition P, Lattice L, const float *grid,
         int lb[3];
         lattice_coords(sc, l, lb[0], lb[1], lb[2]);
         const int bc[3] = {(lb[0] + L.origin) * 4, (lb[1] + L.origin) * 4, (lb[2] + L.origin) * 4};
+        // A part without a particle near a face does not need the velocities, but few parts have none, and
+        // to wait for that knowledge puts two more loads into the chain (256 scenes, 77,514 blocks: 207 ->
+        // 173 us, the 65k cube 9.9 -> 8.8, the dam 47.8 -> 46.4; the fused pass's, with more registers in
+        // use, went from 211 to 247 and still waits).
+        constexpr bool EARLY = !FUSED;
+        BlockNodes<NT> nodes;
+        if (EARLY) block_nodes_ids(nodes, P.lat_gid, l, nb, nb2);
         // speed bound over the stencils of this block's particles (grid blocks lb + {0,1}^3)
         float v2 = 0.0f;
+        int32_t gid[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int32_t gid = P.lat_gid[l + (e >> 2) * nb2 + ((e >> 1) & 1) * nb + (e & 1)];
-            v2 = fmaxf(v2, gid >= 0 ? gvmax[gid] : __builtin_inff());
-        }
+        for (int e = 0; e < 8; ++e) gid[e] = P.lat_gid[l + (e >> 2) * nb2 + ((e >> 1) & 1) * nb + (e & 1)];
+        if (EARLY) block_nodes_load(nodes, grid);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v2 = fmaxf(v2, gid[e] >= 0 ? gvmax[gid[e]] : __builtin_inff());
         const float reach = AFLIP ? __builtin_inff() : sqrtf(v2) * (sc.dt * sc.dxinv) * 1.001f;  // cells (upper bound)
-        bool staged = false;  // grid velocities in LDS: only once a particle needs them
         if (t < 32) s_run[t] = 0u;
         if (t == 0) {
             s_nlist = 0u;
             s_mrun = 0u;
+        }
+        bool staged = EARLY;
+        if (EARLY) block_nodes_stage(nodes, s_v);
+        if (AFLIP) {
+            block_nodes_load(nodes, gstar);
+            block_nodes_stage(nodes, s_vs);
         }
         __syncthreads();
         // segments of up to kMoveList particles: kept particles get direction 13, the
@@ -2021,9 +2034,8 @@ k_g2p_move(State A, Partition P, Lattice L, const float *grid,
             }
             __syncthreads();
             const uint32_t nl = s_nlist;
-            if (nl > 0u && !staged) {  // uniform: nl was read after the barrier
+            if (!EARLY && nl > 0u && !staged) {  // uniform: nl was read after the barrier
                 stage_block_velocity<NT>(s_v, grid, P.lat_gid, l, nb, nb2);
-                if (AFLIP) stage_block_velocity<NT>(s_vs, gstar, P.lat_gid, l, nb, nb2);
                 staged = true;
                 __syncthreads();
             }
@@ -2195,7 +2207,8 @@ struct UpdateArgs {
 // beta.  With u.nonaffine, FLIP (Transfer.cu:1215-1250): the velocity gradient
 // sum vstar_i grad W_i^T in place of C for F (C itself is kept), beta 0.
 template <bool SCATTER, int NT, bool AFLIP = false>
-__global__ void __launch_bounds__(NT) k_g2p_update(UpdateArgs u) {
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(AFLIP ? 2 : 4)))
+k_g2p_update(UpdateArgs u) {
     __shared__ float4 s_v[kTileNodes];
     __shared__ float4 s_vs[AFLIP ? kTileNodes : 1];
     __shared__ uint32_t s_base[32];
@@ -2228,23 +2241,40 @@ __global__ void __launch_bounds__(NT) k_g2p_update(UpdateArgs u) {
         lattice_coords(sc, l, lb[0], lb[1], lb[2]);
         const int bc[3] = {(lb[0] + u.L.origin) * 4, (lb[1] + u.L.origin) * 4, (lb[2] + u.L.origin) * 4};
         const int64_t nb = sc.nb, nb2 = nb * nb;
-        if (SCATTER && t < 64) {
-            // the directions in which this block's particles leave (pass 1's counts)
-            const bool act = t < kDirs && u.cnt27[(int64_t)pr.p * kDirs + t] != 0u;
-            const uint64_t mask = __ballot(act);
-            if (act) s_dir[__popcll(mask & ((1ull << t) - 1ull))] = (uint32_t)t;
-            if (t == 0) s_nact = (uint32_t)__popcll(mask);
+        // The destinations' chain (counts, neighbours' ids, their counts, the new starts) and the
+        // staging's (block ids, values) run side by side: each load is issued as soon as what it needs
+        // is there, and the velocities wait in registers.  (One after the other: 77,514 blocks 375 us, the
+        // dam 124, the tank 26.2; this way 346, 120, 25.6.)
+        constexpr bool EARLY = !(AFLIP && NT == 64);  // that one has no registers left for it
+        BlockNodes<NT> nodes;
+        if (EARLY) block_nodes_ids(nodes, u.lat_gid, l, nb, nb2);
+        if (SCATTER) {
+            if (t < 64) {
+                // the directions in which this block's particles leave (pass 1's counts)
+                const bool act = t < kDirs && u.cnt27[(int64_t)pr.p * kDirs + t] != 0u;
+                const uint64_t mask = __ballot(act);
+                if (act) s_dir[__popcll(mask & ((1ull << t) - 1ull))] = (uint32_t)t;
+                if (t == 0) s_nact = (uint32_t)__popcll(mask);
+            }
+            __syncthreads();
         }
-        stage_block_velocity<NT>(s_v, u.grid, u.lat_gid, l, nb, nb2);
-        if (AFLIP) stage_block_velocity<NT>(s_vs, u.gstar, u.lat_gid, l, nb, nb2);
+        if (EARLY) block_nodes_load(nodes, u.grid);
+        const int n_act = SCATTER ? (int)s_nact : 0;
+        uint32_t dest0 = 0u;
+        if (SCATTER) {
+            move_base_pairs<NT>(l, lb, sc.nb, u.lat_pid, u.lat_xf, u.cnt27, u.parts, nx, s_dir, n_act, s_pair);
+            if (t < n_act) dest0 = move_dest_start((int)s_dir[t], l, lb, sc.nb, u.n_lat_pid, u.n_pblk_start);
+        }
+        if (EARLY) block_nodes_stage(nodes, s_v);
+        else stage_block_velocity<NT>(s_v, u.grid, u.lat_gid, l, nb, nb2);
+        if (AFLIP && EARLY) {
+            block_nodes_load(nodes, u.gstar);
+            block_nodes_stage(nodes, s_vs);
+        } else if (AFLIP) {
+            stage_block_velocity<NT>(s_vs, u.gstar, u.lat_gid, l, nb, nb2);
+        }
         __syncthreads();
         if (SCATTER) {
-            const int n_act = (int)s_nact;
-            move_base_pairs<NT>(l, lb, sc.nb, u.lat_pid, u.lat_xf, u.cnt27, u.parts, nx, s_dir, n_act, s_pair);
-            const uint32_t dest0 = t < n_act ? move_dest_start((int)s_dir[t], l, lb, sc.nb, u.n_lat_pid,
-                                                                 u.n_pblk_start)
-                                             : 0u;
-            __syncthreads();
             if (t < n_act) {
                 uint32_t base = dest0;
 #pragma unroll

@@ -177,14 +177,54 @@ __device__ __forceinline__ int tile_slot(int x, int y, int z) {
 __device__ __forceinline__ int tile_slot_of(int k) { return tile_slot(k / 36, (k / 6) % 6, k % 6); }
 
 // Grid velocities of one particle block's 6^3 stencil region, one float4 (v, 0)
-// per node so a z-run of 3 nodes is 3 contiguous 16-byte LDS reads.
+// per node so a z-run of 3 nodes is 3 contiguous 16-byte LDS reads: at once
+// (stage_block_velocity), or in three steps (block ids, their values, LDS), each a
+// load's latency after the one before, between which a caller puts other loads.
+template <int NT>
+struct BlockNodes {
+    static constexpr int K = (kTileNodes + NT - 1) / NT;  // nodes per thread
+    int32_t at[K];  // the node's grid block, < 0: none
+    float v[K][3];
+};
+template <int NT>
+__device__ __forceinline__ void block_nodes_ids(BlockNodes<NT> &r, const int32_t *lat_gid, int64_t l, int64_t nb,
+                                                int64_t nb2) {
+#pragma unroll
+    for (int q = 0; q < BlockNodes<NT>::K; ++q) {
+        const int k = min((int)threadIdx.x + q * NT, kTileNodes - 1);
+        const int tx = k / 36, ty = (k / 6) % 6, tz = k % 6;
+        r.at[q] = lat_gid[l + (tx >> 2) * nb2 + (ty >> 2) * nb + (tz >> 2)];
+    }
+}
+template <int NT>
+__device__ __forceinline__ void block_nodes_load(BlockNodes<NT> &r, const float *grid) {
+#pragma unroll
+    for (int q = 0; q < BlockNodes<NT>::K; ++q) {
+        const int k = min((int)threadIdx.x + q * NT, kTileNodes - 1);
+        const int tx = k / 36, ty = (k / 6) % 6, tz = k % 6;
+        const int cell = ((tx & 3) * 4 + (ty & 3)) * 4 + (tz & 3);
+        const float *gv = grid + (int64_t)max(r.at[q], 0) * 256 + 64 + cell;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) r.v[q][c] = gv[c * 64];
+    }
+}
+template <int NT>
+__device__ __forceinline__ void block_nodes_stage(const BlockNodes<NT> &r, float4 *s_v) {
+#pragma unroll
+    for (int q = 0; q < BlockNodes<NT>::K; ++q) {
+        const int k = (int)threadIdx.x + q * NT;
+        if (k < kTileNodes)
+            s_v[k] = r.at[q] >= 0 ? make_float4(r.v[q][0], r.v[q][1], r.v[q][2], 0.0f)
+                                  : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+}
 template <int NT = kThreads>
 __device__ __forceinline__ void stage_block_velocity(float4 *s_v, const float *grid, const int32_t *lat_gid, int64_t l,
                                                      int64_t nb, int64_t nb2) {
+    // one node at a time: the callers are short of registers
     for (int k = threadIdx.x; k < kTileNodes; k += NT) {
         const int tx = k / 36, ty = (k / 6) % 6, tz = k % 6;
-        const int ex = tx >> 2, ey = ty >> 2, ez = tz >> 2;
-        const int32_t g = lat_gid[l + ex * nb2 + ey * nb + ez];
+        const int32_t g = lat_gid[l + (tx >> 2) * nb2 + (ty >> 2) * nb + (tz >> 2)];
         const int cell = ((tx & 3) * 4 + (ty & 3)) * 4 + (tz & 3);
         const float *gv = grid + (int64_t)(g >= 0 ? g : 0) * 256 + 64 + cell;
         const float v0 = gv[0], v1 = gv[64], v2 = gv[128];
