@@ -866,19 +866,16 @@ k_p2g(State A, Partition P, Lattice L, const DevMaterial *mats,
                 if (valid && rank[r] == 0) s_wcnt[r * 3 + w][cell[r]] = (uint32_t)__popcll(match);
             }
             __syncthreads();
-            if (w == 0) {
+            // the cells' starts and, from the first chunk, phase B's task order, on a wave each
+            if (w < 2) {
                 uint32_t tot = 0;
 #pragma unroll
                 for (int k = 0; k < kP2GRounds * 3; ++k) tot += s_wcnt[k][lane];
-                uint32_t inc = tot;
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) {
-                    const uint32_t y = __shfl_up(inc, off, 64);
-                    if (lane >= off) inc += y;
-                }
-                s_cstart[lane] = inc - tot;
-                if (lane == 63) s_cstart[64] = inc;
-                if (c0 == ps) {
+                if (w == 0) {
+                    const uint32_t inc = wave_scan_u32(tot);
+                    s_cstart[lane] = inc - tot;
+                    if (lane == 63) s_cstart[64] = inc;
+                } else if (c0 == ps) {
                     // the 192 (cell, x-offset) tasks of phase B sorted by the cell's particle
                     // count, descending (ties by cell), so each wave gets cells of similar
                     // counts and its loop runs close to its own lanes' work
