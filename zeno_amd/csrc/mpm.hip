@@ -798,16 +798,24 @@ __device__ __forceinline__ void p2g_chunk_tail(float *s_pl, const uint8_t *s_tas
 // phases C and D on their own, p2g_chunk_tail); otherwise the registers carry each
 // task's sums from one chunk to the next and phases C and D run once per block.
 // The two agree bit for bit on blocks of at most kP2GChunk particles.
-template <int MODE, bool PP = false, bool FLUSH = false>
-__global__ void __launch_bounds__(kP2GThreads) __attribute__((amdgpu_waves_per_eu(5)))
-k_p2g(State A, Partition P, Lattice L, const DevMaterial *mats,
-                                                     const float *sig, int64_t sig_stride, float *tiles, DevStatus *st,
-                                                     AdjScatter adj, uint32_t skip_upto) {
-    __shared__ float s_pl[kPL * kP2GChunk];
-    static_assert(3 * kTileNodes * 4 <= kPL * kP2GChunk, "tiles alias the payload");
-    __shared__ uint32_t s_wcnt[kP2GRounds * 3][64];
-    __shared__ uint32_t s_cstart[65];
-    __shared__ uint8_t s_task[3 * 64];  // phase B task p -> cell (x-offset p % 3)
+struct P2GShared {
+    float pl[kPL * kP2GChunk];
+    uint32_t wcnt[kP2GRounds * 3][64];
+    uint32_t cstart[65];
+    uint8_t task[3 * 64];  // phase B task p -> cell (x-offset p % 3)
+};
+static_assert(3 * kTileNodes * 4 <= kPL * kP2GChunk, "tiles alias the payload");
+
+// The parts first, first + stride, ... of the partition.
+template <int MODE, bool PP, bool FLUSH>
+__device__ __forceinline__ void p2g_parts(P2GShared &sh, uint32_t first, uint32_t stride, State A,
+                                          const Partition &P, const Lattice &L, const DevMaterial *mats,
+                                          const float *sig, int64_t sig_stride, float *tiles, DevStatus *st,
+                                          const AdjScatter &adj, uint32_t skip_upto) {
+    float *s_pl = sh.pl;
+    uint32_t(&s_wcnt)[kP2GRounds * 3][64] = sh.wcnt;
+    uint32_t *s_cstart = sh.cstart;
+    uint8_t *s_task = sh.task;
 
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const uint32_t nblocks = P.counts[0], nx = P.counts[2];
@@ -818,7 +826,7 @@ k_p2g(State A, Partition P, Lattice L, const DevMaterial *mats,
     s_task[t] = (uint8_t)(t / 3);
 
     // one part per iteration, into its own tile
-    for (uint32_t j = blockIdx.x; j < nblocks + nx; j += gridDim.x) {
+    for (uint32_t j = first; j < nblocks + nx; j += stride) {
         const PartRef pr = part_ref(V, j, nblocks);
         const uint32_t b = pr.b;
         // k_p2g_sparse takes the blocks of at most skip_upto particles (a single part)
@@ -957,6 +965,37 @@ k_p2g(State A, Partition P, Lattice L, const DevMaterial *mats,
     if (mismatch) atomicOr(&st->bin_mismatch, 1u);
 }
 
+template <int MODE, bool PP = false, bool FLUSH = false>
+__global__ void __launch_bounds__(kP2GThreads) __attribute__((amdgpu_waves_per_eu(5)))
+k_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t sig_stride, float *tiles,
+      DevStatus *st, AdjScatter adj, uint32_t skip_upto) {
+    __shared__ P2GShared sh;
+    p2g_parts<MODE, PP, FLUSH>(sh, blockIdx.x, gridDim.x, A, P, L, mats, sig, sig_stride, tiles, st, adj, skip_upto);
+}
+
+// The two scatters of a FLIP transfer, MODE into tiles and MODE2 into tiles2, as one launch: half the
+// workgroups each.  Neither reads what the other writes, and a launch over few parts takes as long as
+// one part does.  Workgroups of one part run on one XCD (numbers equal modulo 8) and share its loads.
+// One launch after the other and as a pair: 30 parts (nine waves each) 11.1 + 11.3 and 12.2 us, 170 parts
+// 12.5 + 13.8 and 18.6, 366 parts 14.1 + 20.1 and 22.0, 576 parts 16.2 + 15.9 and 19.5, 5,800 parts 65 +
+// 67 and 119.
+__device__ __forceinline__ bool pair_unit(uint32_t &first, uint32_t &stride) {
+    first = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u);
+    stride = gridDim.x >> 1;
+    return (blockIdx.x & 8u) != 0u;
+}
+template <int MODE, int MODE2, bool PP>
+__global__ void __launch_bounds__(kP2GThreads) __attribute__((amdgpu_waves_per_eu(5)))
+k_p2g_pair(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t sig_stride,
+           float *tiles, float *tiles2, DevStatus *st) {
+    __shared__ P2GShared sh;
+    uint32_t first, stride;
+    if (!pair_unit(first, stride))
+        p2g_parts<MODE, PP, false>(sh, first, stride, A, P, L, mats, sig, sig_stride, tiles, st, AdjScatter{}, 0u);
+    else
+        p2g_parts<MODE2, PP, false>(sh, first, stride, A, P, L, mats, sig, sig_stride, tiles2, st, AdjScatter{}, 0u);
+}
+
 // P2G of few parts: k_p2g's sums, bit for bit, with nine waves a part, for launches whose parts do
 // not fill the chip, where a part's chain of dependent steps is the launch's time.  Thread =
 // particle for the payload (576 a chunk, so a block at 8 per cell needs one; every field loaded at
@@ -964,17 +1003,23 @@ k_p2g(State A, Partition P, Lattice L, const DevMaterial *mats,
 // instead of nine.  A node's additions are those of k_p2g in its order: the particles of a cell one
 // after another, across the chunks in registers; the cells' sums into the x-offset's tile by
 // (oy, oz), where one wave holds all of an (ox, oy), so only the three oy are a barrier apart.
-// Launches of 35 and 180 parts: 17.9 -> 12.9 and 17.8 -> 13.7 us; 366 parts (more than the CUs):
-// 14.7 -> 16.6, 576: 16.4 -> 26, as the threads' weights are formed nine times, not three.
+// Launches of 35 and 180 parts: 17.9 -> 12.9 and 17.8 -> 13.7 us; 388 and 430 parts (more than the
+// CUs): 18.7 -> 21.5 and 19.8 -> 23.5, as the threads' weights are formed nine times, not three.
 constexpr int kWideThreads = 576;
 constexpr int kWideWaves = kWideThreads / 64;
+struct P2GWideShared {
+    float pl[kPL * kWideThreads];
+    float4 tile[3 * kTileNodes];
+    uint32_t wcnt[kWideWaves][64];
+};
 template <int MODE, bool PP>
-__global__ void __launch_bounds__(kWideThreads)
-k_p2g_wide(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t sig_stride,
-           float *tiles, DevStatus *st, AdjScatter adj) {
-    __shared__ float s_pl[kPL * kWideThreads];
-    __shared__ float4 s_tile[3 * kTileNodes];
-    __shared__ uint32_t s_wcnt[kWideWaves][64];
+__device__ __forceinline__ void p2g_wide_parts(P2GWideShared &sh, uint32_t first, uint32_t stride, State A,
+                                               const Partition &P, const Lattice &L, const DevMaterial *mats,
+                                               const float *sig, int64_t sig_stride, float *tiles, DevStatus *st,
+                                               const AdjScatter &adj) {
+    float *s_pl = sh.pl;
+    float4 *s_tile = sh.tile;
+    uint32_t(&s_wcnt)[kWideWaves][64] = sh.wcnt;
 
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -984,7 +1029,7 @@ k_p2g_wide(State A, Partition P, Lattice L, const DevMaterial *mats, const float
     const uint32_t nblocks = P.counts[0], nx = P.counts[2];
     const PartView V = part_view(P, L.part_shift);
     bool mismatch = false;
-    for (uint32_t j = blockIdx.x; j < nblocks + nx; j += gridDim.x) {
+    for (uint32_t j = first; j < nblocks + nx; j += stride) {
         const PartRef pr = part_ref(V, j, nblocks);
         const uint32_t b = pr.b, ps = pr.lo, pe = pr.hi;
         const SceneParams sc = scene_params(L, L.nscenes == 1 ? 0u : P.pblk_scene[b]);
@@ -1151,6 +1196,27 @@ k_p2g_wide(State A, Partition P, Lattice L, const DevMaterial *mats, const float
         __syncthreads();
     }
     if (mismatch) atomicOr(&st->bin_mismatch, 1u);
+}
+
+template <int MODE, bool PP>
+__global__ void __launch_bounds__(kWideThreads)
+k_p2g_wide(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t sig_stride,
+           float *tiles, DevStatus *st, AdjScatter adj) {
+    __shared__ P2GWideShared sh;
+    p2g_wide_parts<MODE, PP>(sh, blockIdx.x, gridDim.x, A, P, L, mats, sig, sig_stride, tiles, st, adj);
+}
+
+// k_p2g_pair with nine waves a part
+template <int MODE, int MODE2, bool PP>
+__global__ void __launch_bounds__(kWideThreads)
+k_p2g_wide_pair(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t sig_stride,
+                float *tiles, float *tiles2, DevStatus *st) {
+    __shared__ P2GWideShared sh;
+    uint32_t first, stride;
+    if (!pair_unit(first, stride))
+        p2g_wide_parts<MODE, PP>(sh, first, stride, A, P, L, mats, sig, sig_stride, tiles, st, AdjScatter{});
+    else
+        p2g_wide_parts<MODE2, PP>(sh, first, stride, A, P, L, mats, sig, sig_stride, tiles2, st, AdjScatter{});
 }
 
 // P2G of the particle blocks holding at most 64 particles (kSparseMax), one wave
@@ -3514,20 +3580,44 @@ void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const 
                            mats, sig, stride, tiles, st);
 }
 
+namespace {
+// Both scatters of a FLIP transfer (as launch_p2g_mode); the grid is a multiple of 16 (pair_unit).
+template <int MODE, int MODE2, bool PP>
+void launch_p2g_pair(int64_t parts, int64_t max_blocks, hipStream_t s, State A, Partition P, Lattice L,
+                     const DevMaterial *mats, const float *sig, int64_t stride, float *tiles, float *tiles2,
+                     DevStatus *st) {
+    const dim3 g(16u * persistent_grid(max_blocks, 8, 1 << 16));
+    if (parts <= kWideMaxParts)
+        hipLaunchKernelGGL((k_p2g_wide_pair<MODE, MODE2, PP>), g, dim3(kWideThreads), 0, s, A, P, L, mats, sig, stride,
+                           tiles, tiles2, st);
+    else
+        hipLaunchKernelGGL((k_p2g_pair<MODE, MODE2, PP>), g, dim3(kP2GThreads), 0, s, A, P, L, mats, sig, stride,
+                           tiles, tiles2, st);
+}
+}  // namespace
+
 void launch_p2g_aflip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
                       float *tiles, float *tiles2, DevStatus *st, int64_t parts, int64_t max_blocks,
                       hipStream_t s) {
     if (max_blocks <= 0) return;
-    launch_p2g_mode<kP2GMomentum>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
-    launch_p2g_mode<kP2GStress>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
+    if (L.pp_mass)
+        launch_p2g_pair<kP2GMomentum, kP2GStress, true>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles,
+                                                        tiles2, st);
+    else
+        launch_p2g_pair<kP2GMomentum, kP2GStress, false>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles,
+                                                        tiles2, st);
 }
 
 void launch_p2g_flip(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
                      float *tiles, float *tiles2, DevStatus *st, int64_t parts, int64_t max_blocks,
                      hipStream_t s) {
     if (max_blocks <= 0) return;
-    launch_p2g_mode<kP2GFlipMomentum>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles, st, AdjScatter{}, 0u);
-    launch_p2g_mode<kP2GFlipStress>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles2, st, AdjScatter{}, 0u);
+    if (L.pp_mass)
+        launch_p2g_pair<kP2GFlipMomentum, kP2GFlipStress, true>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles,
+                                                        tiles2, st);
+    else
+        launch_p2g_pair<kP2GFlipMomentum, kP2GFlipStress, false>(parts, max_blocks, s, A, P, L, mats, sig, stride, tiles,
+                                                        tiles2, st);
 }
 
 void launch_grid_aflip(int mode, Partition P, Lattice L, const float *tiles, const float *tiles2, float *grid,
