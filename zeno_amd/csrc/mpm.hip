@@ -521,6 +521,17 @@ __device__ __forceinline__ void plastic_project(const DevMaterial &mt, float F[3
     }
 }
 
+// The stress term of fixed corotated without a fiber: f_stress_term's branch, operation for operation.
+__device__ __forceinline__ void fcr_stress_term(float s, float mu, float lam, const float F[3][3], float out[3][3]) {
+    float Pk[3][3];
+    fcr_piola(F, mu, lam, Pk);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            out[r][c] = (s * Pk[r][0]) * F[c][0] + (s * Pk[r][1]) * F[c][1] + (s * Pk[r][2]) * F[c][2];
+}
+
 // Stress term of the F-based particles, one lane per particle (f_stress_term).
 // Computed apart from P2G so that these registers and run times do not hold
 // back the transfer's workgroups; J-fluid particles are skipped (P2G forms
@@ -551,14 +562,8 @@ __global__ void __launch_bounds__(kThreads) k_stress(State A, int64_t n, Lattice
                 for (int c = 0; c < 3; ++c) fa[c] = chan(A.ch, i, kChFiber + c);
             }
             f_stress_term(mt, s, mu, lam, F, fa, out);
-        } else {  // f_stress_term's fixed-corotated branch, operation for operation
-            float Pk[3][3];
-            fcr_piola(F, mu, lam, Pk);
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-                    out[r][c] = (s * Pk[r][0]) * F[c][0] + (s * Pk[r][1]) * F[c][1] + (s * Pk[r][2]) * F[c][2];
+        } else {
+            fcr_stress_term(s, mu, lam, F, out);
         }
 #pragma unroll
         for (int q9 = 0; q9 < 9; ++q9) sig[q9 * stride + k] = out[q9 / 3][q9 % 3];
@@ -1012,7 +1017,11 @@ struct P2GWideShared {
     float4 tile[3 * kTileNodes];
     uint32_t wcnt[kWideWaves][64];
 };
-template <int MODE, bool PP>
+// STRESS: forms the stress term itself (fixed corotated and J-fluid only, kP2GForward), as k_stress does,
+// between the ranking and its barrier, and reads F where it would read the term: no launch of k_stress,
+// 3.8 to 4.7 us and the gap after it, for 0.5 to 2.5 us more here (35, 180 parts: 12.1 + 3.8 -> 12.8,
+// 13.2 + 4.7 -> 15.7).
+template <int MODE, bool PP, bool STRESS = false>
 __device__ __forceinline__ void p2g_wide_parts(P2GWideShared &sh, uint32_t first, uint32_t stride, State A,
                                                const Partition &P, const Lattice &L, const DevMaterial *mats,
                                                const float *sig, int64_t sig_stride, float *tiles, DevStatus *st,
@@ -1053,6 +1062,11 @@ __device__ __forceinline__ void p2g_wide_parts(P2GWideShared &sh, uint32_t first
             for (int k = 0; k < 3; ++k) xp[k] = run_chan(run, off, k);
             P2GIn in;
             if (MODE != kP2GAdjoint) p2g_load(A, run, off, in, PP);
+            float sg[3][3];  // F, then the stress term
+            if (STRESS) {
+#pragma unroll
+                for (int q = 0; q < 9; ++q) sg[q / 3][q % 3] = run_chan(run, off, kChF + q);
+            }
             float fr[3];
             int lc[3];
 #pragma unroll
@@ -1070,6 +1084,16 @@ __device__ __forceinline__ void p2g_wide_parts(P2GWideShared &sh, uint32_t first
             s_wcnt[w][lane] = 0u;
             wave_lds_order();
             if (valid && rank == 0u) s_wcnt[w][cell] = (uint32_t)__popcll(match);
+            if (STRESS && (in.mw & kMatF)) {
+                const DevMaterial &mt = mats[in.mw & kMatIndexMask];
+                const float vs = (-sc.dt * sc.Dinv) * (PP ? run_chan(run, off, kChVol) : mt.vol);
+                const float mu = L.pp_lame ? run_chan(run, off, kChMu) : mt.mu;
+                const float lam = L.pp_lame ? run_chan(run, off, kChLam) : mt.lam;
+                float F[3][3];
+#pragma unroll
+                for (int q = 0; q < 9; ++q) F[q / 3][q % 3] = sg[q / 3][q % 3];
+                fcr_stress_term(vs, mu, lam, F, sg);
+            }
             __syncthreads();
             uint32_t tot = 0u, before = 0u;
 #pragma unroll
@@ -1100,6 +1124,8 @@ __device__ __forceinline__ void p2g_wide_parts(P2GWideShared &sh, uint32_t first
                     }
                 } else if (MODE == kP2GFlipStress) {
                     p2g_payload_flip_stress<kWideThreads>(in, i, mats, sig, sig_stride, dx, sc.dt, fr, pl);
+                } else if (STRESS) {
+                    p2g_payload_f<kWideThreads>(in, i, mats, [&](int q) { return sg[q / 3][q % 3]; }, dx, sdt, fr, pl);
                 } else {
                     p2g_payload<kWideThreads, MODE == kP2GMomentum       ? 1
                                               : MODE == kP2GStress       ? 2
@@ -1198,12 +1224,12 @@ __device__ __forceinline__ void p2g_wide_parts(P2GWideShared &sh, uint32_t first
     if (mismatch) atomicOr(&st->bin_mismatch, 1u);
 }
 
-template <int MODE, bool PP>
+template <int MODE, bool PP, bool STRESS = false>
 __global__ void __launch_bounds__(kWideThreads)
 k_p2g_wide(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t sig_stride,
            float *tiles, DevStatus *st, AdjScatter adj) {
     __shared__ P2GWideShared sh;
-    p2g_wide_parts<MODE, PP>(sh, blockIdx.x, gridDim.x, A, P, L, mats, sig, sig_stride, tiles, st, adj);
+    p2g_wide_parts<MODE, PP, STRESS>(sh, blockIdx.x, gridDim.x, A, P, L, mats, sig, sig_stride, tiles, st, adj);
 }
 
 // k_p2g_pair with nine waves a part
@@ -3534,10 +3560,14 @@ void launch_stress(State A, int64_t n, Lattice L, const DevMaterial *mats, float
         hipLaunchKernelGGL(k_stress<false>, dim3(grid_for(n, 2048)), dim3(kThreads), 0, s, A, n, L, mats, sig, stride);
 }
 
+constexpr int64_t kWideMaxParts = 256;  // launch_p2g_mode
+bool p2g_forms_stress(int64_t parts, bool sparse, bool flush, bool general) {
+    return !sparse && !flush && !general && parts <= kWideMaxParts;
+}
+
 // P2G over about `parts` parts (max_blocks: the bound that sizes the grid): k_p2g_wide up to the
 // chip's 256 CUs, where its shorter chain is the launch's time (figures at the kernel), k_p2g above.
 // The two give the same bits.
-constexpr int64_t kWideMaxParts = 256;
 template <int MODE>
 void launch_p2g_mode(int64_t parts, int64_t max_blocks, hipStream_t s, State A, Partition P, Lattice L, const DevMaterial *mats,
                      const float *sig, int64_t stride, float *tiles, DevStatus *st, AdjScatter adj,
@@ -3562,9 +3592,18 @@ void launch_p2g_mode(int64_t parts, int64_t max_blocks, hipStream_t s, State A, 
 
 void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
                 float *tiles, DevStatus *st, int64_t parts, int64_t max_blocks, hipStream_t s, bool sparse,
-                bool flush) {
+                bool flush, bool stress) {
     if (max_blocks <= 0) return;
     const dim3 g(persistent_grid(max_blocks, 1, 1 << 20));
+    if (stress) {
+        if (L.pp_mass)
+            hipLaunchKernelGGL((k_p2g_wide<kP2GForward, true, true>), g, dim3(kWideThreads), 0, s, A, P, L, mats, sig,
+                               stride, tiles, st, AdjScatter{});
+        else
+            hipLaunchKernelGGL((k_p2g_wide<kP2GForward, false, true>), g, dim3(kWideThreads), 0, s, A, P, L, mats, sig,
+                               stride, tiles, st, AdjScatter{});
+        return;
+    }
     // with sparse, blocks of <= kSparseMax particles go to the one-wave kernel (one chunk either way)
     const uint32_t skip = sparse ? (uint32_t)kSparseMax : 0u;
     if (!flush)

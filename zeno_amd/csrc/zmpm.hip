@@ -815,21 +815,23 @@ int32_t zmpm_p2g(zmpm_ctx *ctx, float dt) {
         ctx->set_device();
         ctx->L.part_shift = ctx->psize[ctx->pcur];  // the parts the partition was cut into
         set_steps(ctx, step_args(dt, nullptr, 0, 0), SET_DT);
-        launch_stress(ctx->st[ctx->cur], ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->stream,
-                      ctx->stress_general());
+        const int64_t np = ctx->parts_now();  // once: the device may update the counts meanwhile
+        const bool sparse = ctx->p2g_sparse(), general = ctx->stress_general();
+        const bool own_stress = !ctx->flip_style() && p2g_forms_stress(np, sparse, ctx->fused_path(), general);
+        if (!own_stress)
+            launch_stress(ctx->st[ctx->cur], ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->stream, general);
         if (ctx->flip_style()) {
             if (ctx->transfer == ZMPM_TRANSFER_FLIP)
                 launch_p2g_flip(ctx->st[ctx->cur], ctx->part[ctx->pcur], ctx->L, ctx->mats, ctx->sig, ctx->cap,
-                                ctx->tiles, ctx->tiles2, ctx->status, ctx->parts_now(), ctx->max_units(), ctx->stream);
+                                ctx->tiles, ctx->tiles2, ctx->status, np, ctx->max_units(), ctx->stream);
             else
                 launch_p2g_aflip(ctx->st[ctx->cur], ctx->part[ctx->pcur], ctx->L, ctx->mats, ctx->sig, ctx->cap,
-                                 ctx->tiles, ctx->tiles2, ctx->status, ctx->parts_now(), ctx->max_units(), ctx->stream);
+                                 ctx->tiles, ctx->tiles2, ctx->status, np, ctx->max_units(), ctx->stream);
             launch_grid_aflip(GRID_COMBINE, ctx->part[ctx->pcur], ctx->L, ctx->tiles, ctx->tiles2, ctx->grid,
                               ctx->gstar, ctx->gvmax, ctx->max_gblocks(), ctx->stream);
         } else {
             launch_p2g(ctx->st[ctx->cur], ctx->part[ctx->pcur], ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles,
-                       ctx->status, ctx->parts_now(), ctx->max_units(), ctx->stream, ctx->p2g_sparse(),
-                       ctx->fused_path());
+                       ctx->status, np, ctx->max_units(), ctx->stream, sparse, ctx->fused_path(), own_stress);
             launch_grid(GRID_COMBINE, ctx->part[ctx->pcur], ctx->L, ctx->tiles, ctx->grid, ctx->gvmax,
                         ctx->max_gblocks(), ctx->stream);
         }
@@ -1176,7 +1178,8 @@ void substep_fused(zmpm_ctx *ctx, hipEvent_t *ev, int grow, bool last) {
     if (!ctx->tiles_valid) launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, ctx->stress_general());
     if (ev) HIP_CHECK(hipEventRecord(ev[1], s));
     if (!ctx->tiles_valid)
-        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, ctx->p2g_sparse(), true);
+        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, ctx->p2g_sparse(),
+                   true, false);
     if (ev) HIP_CHECK(hipEventRecord(ev[2], s));
     launch_grid(grid_mode, P, ctx->L, ctx->tiles, ctx->grid, ctx->gvmax, ngb, s, nullptr, ctx->vmax, ctx->L.nscenes);
     launch_colliders(P, ctx->L, ctx->grid, ctx->gvmax, ngb, true, s);
@@ -1223,7 +1226,7 @@ void fused_prologue(zmpm_ctx *ctx, bool force = false) {
     const Partition P = ctx->part[ctx->pcur];
     launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->stream, ctx->stress_general());
     launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, ctx->parts_now(), ctx->max_units(),
-               ctx->stream, ctx->p2g_sparse(), true);
+               ctx->stream, ctx->p2g_sparse(), true, false);
     ctx->tiles_valid = true;
 }
 
@@ -1240,8 +1243,10 @@ void substep_once(zmpm_ctx *ctx, hipEvent_t *ev, int grow = 0, bool last = true)
     const int64_t np = ctx->parts_now();
     const int64_t npb = grown(ctx->max_units(), grow), ngb = grown(ctx->max_gblocks(), grow);
     ctx->tiles_valid = false;
+    const bool sparse = ctx->p2g_sparse(), general = ctx->stress_general();
+    const bool own_stress = !ctx->flip_style() && p2g_forms_stress(np, sparse, false, general);
     if (ev) HIP_CHECK(hipEventRecord(ev[0], s));
-    launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, ctx->stress_general());
+    if (!own_stress) launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, general);
     if (ev) HIP_CHECK(hipEventRecord(ev[1], s));
     // FLIP transfers: momentum and stress apart, velocities v and vstar
     const bool aflip = ctx->flip_style(), nonaffine = ctx->transfer == ZMPM_TRANSFER_FLIP;
@@ -1251,7 +1256,8 @@ void substep_once(zmpm_ctx *ctx, hipEvent_t *ev, int grow = 0, bool last = true)
     else if (aflip)
         launch_p2g_aflip(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->tiles2, ctx->status, np, npb, s);
     else
-        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, ctx->p2g_sparse());
+        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, sparse, false,
+                   own_stress);
     if (ev) HIP_CHECK(hipEventRecord(ev[2], s));
     if (aflip)
         launch_grid_aflip(grid_mode, P, ctx->L, ctx->tiles, ctx->tiles2, ctx->grid, gstar, ctx->gvmax, ngb, s,
@@ -1567,9 +1573,11 @@ int32_t zmpm_adjoint_substep(zmpm_ctx *ctx, const zmpm_step_params *p, const zmp
         const int64_t np = ctx->parts_now(), npb = ctx->max_units(), ngb = ctx->max_gblocks();
         AdjArrays aa{adj->x, adj->v, adj->C, adj->F, adj->mu, adj->lam, adj->n};
         // forward transfer again: combined mass and momentum in grid, updated velocities in grid_v
-        launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, ctx->stress_general());
-        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, ctx->p2g_sparse(),
-                   ctx->fused_path());
+        const bool sparse = ctx->p2g_sparse(), general = ctx->stress_general();
+        const bool own_stress = p2g_forms_stress(np, sparse, ctx->fused_path(), general);
+        if (!own_stress) launch_stress(A, ctx->n, ctx->L, ctx->mats, ctx->sig, ctx->cap, s, general);
+        launch_p2g(A, P, ctx->L, ctx->mats, ctx->sig, ctx->cap, ctx->tiles, ctx->status, np, npb, s, sparse,
+                   ctx->fused_path(), own_stress);
         launch_grid(GRID_COMBINE | GRID_KEEP | GRID_UPDATE | GRID_BOUNDARY, P, ctx->L, ctx->tiles, ctx->grid,
                     ctx->gvmax, ngb, s, ctx->grid_v);
         // G2P adjoint: particle part, then its velocity scatter into gbar

@@ -250,8 +250,11 @@ void launch_stress(State A, int64_t n, Lattice L, const DevMaterial *mats, float
 // sparse: blocks of at most 64 particles go to a one-wave-per-block kernel (a second launch).
 // flush: the fused pass's chunk-flush grouping of blocks of more than one chunk (k_p2g FLUSH)
 void launch_p2g(State A, Partition P, Lattice L, const DevMaterial *mats, const float *sig, int64_t stride,
-                float *tiles, DevStatus *st, int64_t parts, int64_t max_blocks, hipStream_t s, bool sparse = false,
-                bool flush = false);
+                float *tiles, DevStatus *st, int64_t parts, int64_t max_blocks, hipStream_t s, bool sparse,
+                bool flush, bool stress);
+// whether launch_p2g can form the stress terms itself (stress), so that launch_stress is not needed:
+// few parts, no material other than fixed corotated and J-fluid, no fiber
+bool p2g_forms_stress(int64_t parts, bool sparse, bool flush, bool general);
 // mode bits for launch_grid
 enum { GRID_COMBINE = 1, GRID_UPDATE = 2, GRID_BOUNDARY = 4, GRID_CLEAR = 8, GRID_KEEP = 16 };
 // gvmax: per grid block max |v|^2, written by GRID_UPDATE
