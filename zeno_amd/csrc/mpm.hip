@@ -3472,6 +3472,11 @@ __global__ void __launch_bounds__(kThreads) k_cell_volume(State A, int64_t n, Pa
 // one atomic max on the float bits per wave whose blocks share a scene, per lane
 // otherwise.  Non-negative floats order as their bits, and max is order
 // independent, so the result is deterministic.
+__global__ void __launch_bounds__(kThreads) k_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb,
+                                                        uint32_t *host) {
+    for (int32_t i = threadIdx.x; i < na + nb; i += kThreads) host[i] = i < na ? a[i] : b[i - na];
+}
+
 __global__ void __launch_bounds__(kThreads) k_reduce_vmax(const float *gvmax, const uint32_t *gblk_scene,
                                                           const uint32_t *counts, uint32_t *out) {
     const uint32_t ng = counts[1];
@@ -3699,6 +3704,10 @@ void launch_grid(int mode, Partition P, Lattice L, const float *tiles, float *gr
     if (max_blocks <= 0) return;
     hipLaunchKernelGGL(k_grid, dim3(persistent_grid(max_blocks, 4, 1 << 20)), dim3(kThreads), 0, s, mode, P, L, tiles,
                        grid, gvmax, out ? out : grid, vclear, nclear);
+}
+
+void launch_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb, uint32_t *host, hipStream_t s) {
+    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(kThreads), 0, s, a, na, b, nb, host);
 }
 
 void launch_reduce_vmax(const float *gvmax, Partition P, int64_t max_blocks, uint32_t *out, hipStream_t s) {

@@ -265,6 +265,8 @@ void launch_grid(int mode, Partition P, Lattice L, const float *tiles, float *gr
                  int32_t nclear = 0);
 // out[scene] = max over the scene's grid blocks of gvmax, as float bits (out zeroed first)
 void launch_reduce_vmax(const float *gvmax, Partition P, int64_t max_blocks, uint32_t *out, hipStream_t s);
+// a[0 .. na), then b[0 .. nb), to host (device-mapped host memory)
+void launch_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb, uint32_t *host, hipStream_t s);
 // G2P pass 1 of the fused substep: direction of each particle's new block, per-block
 // direction counts, destination marks.  Also resets the lattice scan's state.
 // wg: threads per workgroup, 64 or 256 (one particle block per workgroup either way)
