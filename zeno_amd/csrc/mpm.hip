@@ -2016,8 +2016,11 @@ k_g2p_move(State A, Partition P, Lattice L, const float *grid,
     __shared__ uint32_t s_nlist;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    // the two jobs of the launch that are no part's go to the last workgroups: past the parts there are
+    // some with nothing else to do (77,514 blocks: 171 -> 165 us)
+    const uint32_t back = gridDim.x - 1u - blockIdx.x;
     {
-        const int64_t gtid = blockIdx.x * (int64_t)NT + t, gsz = (int64_t)gridDim.x * NT;
+        const int64_t gtid = back * (int64_t)NT + t, gsz = (int64_t)gridDim.x * NT;
         for (int64_t k = gtid; k < B.scan_tiles; k += gsz) {
             B.scan_p.status[k] = 0ull;
             B.scan_g.status[k] = 0ull;
@@ -2030,7 +2033,7 @@ k_g2p_move(State A, Partition P, Lattice L, const float *grid,
     // order free, so deterministic)
     if (B.vmax_out) {
         const uint32_t ng = P.counts[1];
-        for (int64_t g0 = blockIdx.x * (int64_t)NT; g0 < ng; g0 += (int64_t)gridDim.x * NT) {  // uniform
+        for (int64_t g0 = back * (int64_t)NT; g0 < ng; g0 += (int64_t)gridDim.x * NT) {  // uniform
             const int64_t g = g0 + t;
             const bool valid = g < ng;
             const uint32_t scene = valid ? (L.nscenes == 1 ? 0u : P.gblk_scene[g]) : 0xffffffffu;
