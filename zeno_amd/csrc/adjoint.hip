@@ -27,8 +27,12 @@ namespace {
 // The two adjoint gathers treat every particle on its own, so a particle block is
 // split over kAdjChunks workgroups of kAdjThreads (each stages the block's grid
 // values): small differentiable scenes have too few blocks to fill the GPU.
-constexpr int kAdjThreads = 64;
-constexpr int kAdjChunks = 8;
+// P2G and G2P adjoint with 8 workgroups of 64, 3 of 192, 2 of 256 and 1 of 512 a block: 131,072 particles
+// 34.5 + 23.9, 26.4 + 17.7, 28.9 + 18.9, 28.0 + 19.5 us; 8 scenes of 5k 22.7 + 16.1, 17.7 + 12.1, 20.5 +
+// 13.9, 18.8 + 13.1; 400,000 65.6 + 48.2, 62.2 + 44.1, 59.8 + 45.6, 59.5 + 47.5; 3,000 10.8 + 7.9, 10.9 +
+// 7.4, 10.8 + 7.3, 12.6 + 9.1 (staging by one wave takes four rounds; a block at 8 per cell is 512).
+constexpr int kAdjThreads = 192;
+constexpr int kAdjChunks = 3;
 
 // d w / d f of the quadratic B-spline weights of bspline_w
 __device__ __forceinline__ void bspline_dw(float f, float dw[3]) {
