@@ -1985,15 +1985,14 @@ constexpr uint32_t kDirStay = 13;
 // than that bound times dt (plus a rounding margin) from its block's faces
 // keeps its block: it gets direction 13 without the gather.  The others (a few
 // per cent at CFL-limited steps) are listed and gathered together, so the
-// 27-node interpolation runs on full waves; a block stages its grid velocities
-// in LDS only when it lists a particle, and a block segment that lists none
+// 27-node interpolation runs on full waves; a block segment that lists none
 // takes its ranks from the particle order without ballots.  Every direction
 // equals the one the full interpolation gives.
 // NT: threads per workgroup (64 or 256; the context's rule or zmpm_autotune).
 // AFLIP: the FLIP transfers (grid velocities v and vstar, the particle's own v
 // blended in, the particle's beta or 0 for non-affine FLIP); every particle is
 // interpolated.
-// amdgpu_waves_per_eu(5): at most 96 VGPRs (the compiler then needs about 70), so more
+// amdgpu_waves_per_eu(5): at most 96 VGPRs (the compiler then needs 74 to 85), so more
 // particle blocks are in flight per CU; the interpolation is rare.
 // FUSED (for the fused G2P / P2G pass, APIC): in place of the codes, the block's
 // stayers (direction 13) are listed in order at B.code[ps + rank] and its movers

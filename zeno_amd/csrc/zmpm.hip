@@ -77,13 +77,13 @@ struct zmpm_ctx {
     // Threads per workgroup (one part each) of the G2P kernels: as zmpm_autotune found, else by how
     // many parts there are.  Few leave wave slots empty, so a part gets as many threads as pay; many
     // fill the chip with one wave each, which waits at no barrier.
-    // Move, 180 parts of 363 particles: 13.8 us with 64 threads, 9.9 with 256, 9.4 with 512; 1,180 of
-    // 340: 16.2, 11.7, 18.0; 1,800 of 340: 16.9, 18.9, 25.3; 9,990 of 420: 48, 71, 131; 82,757 of 60:
-    // 207, 345, -.  Update, the same: 22.2, 12.2, 10.5; 27.2, 19.2, 22.2; 27.1, 26.8, 32.3; 128, 124,
-    // 160; 375, 517, -; about 400 parts: 24.1, 13.5, 12.1; 740: 26.1, 16.4, 19.1.
+    // Move, 180 parts of 363 particles: 12.4 us with 64 threads, 8.4 with 256, 8.2 with 512; 1,180 of
+    // 340: 15.1, 10.8, 16.9; 1,800 of 340: 16.5, 17.7, 24.2; 9,990 of 420: 46, 67, 114; 77,514 of 60:
+    // 165, 319, -.  Update, the same: 22.1, 12.4, 10.8; 27.8, 19.0, 21.7; 27.8, 25.5, 30.4; 127, 119,
+    // 153; 340, 506, -; about 400 parts: 24.9, 14.1, 13.0; 740: 26.5, 16.4, 18.4.
     // FLIP transfers (the particles are all interpolated, twice the registers), move and update, 366
-    // parts: 27 and 51 with 64, 16 and 22 with 256, 15 and 24 with 512; 1,750: 37 and 46, 29 and 47, 35
-    // and 58; 5,800: 88 and 176, 68 and 156, 97 and 183.
+    // parts: 27 and 34 with 64, 16 and 16 with 256, 15 and 19 with 512; 1,750: 37 and 44, 28 and 44, 34
+    // and 54; 5,800: 87 and 159, 68 and 144, 95 and 170.
     int wg_move_tuned = 0, wg_update_tuned = 0;
     bool many_small_parts() const { return parts_now() >= 1536 && n <= 96 * parts_now(); }
     int wg_move() const {
@@ -96,7 +96,7 @@ struct zmpm_ctx {
     }
     // one-wave P2G for blocks of <= 64 particles, a launch of its own: as zmpm_autotune found, else
     // where the chip is full of blocks that hold few particles.  (A launch that finds no such block
-    // still costs 13-18 us; on 82,757 blocks of 60 particles on average it gains 423 against 440 us.)
+    // still costs 13-18 us; on 77,514 blocks of 60 particles on average it gains 423 against 440 us.)
     int p2g_sparse_tuned = -1;
     bool p2g_sparse() const {
         if (p2g_sparse_tuned >= 0) return p2g_sparse_tuned != 0;
