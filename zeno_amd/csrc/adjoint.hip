@@ -154,30 +154,27 @@ __global__ void __launch_bounds__(kAdjThreads) k_g2p_adjoint(State A, Partition 
             float dw[3][3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) bspline_dw(ar.f[k], dw[k]);
-            // line by line along z: s = v_i . t with t = a + B d advanced by B's last column, then the sums
-            // of s w_z and s w'_z into the three directions
-            float gx[3] = {0.0f, 0.0f, 0.0f}, tz[3];
-#pragma unroll
-            for (int r = 0; r < 3; ++r) tz[r] = Bq[r][2] * sc.dx;
+            // line by line along z: s = v_i . t with t = a + B d, of which only B's last column changes along
+            // the line, then the sums of s w_z and s w'_z into the three directions
+            float gx[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll 1
             for (int ox = 0; ox < 3; ++ox) {
                 const float wx = pick3(ar.w[0], ox), dwx = pick3(dw[0], ox), d0 = ((float)ox - ar.f[0]) * sc.dx;
                 float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;  // sums over y of w_y S, w'_y S, w_y S'
 #pragma unroll
                 for (int oy = 0; oy < 3; ++oy) {
-                    const float d1 = ((float)oy - ar.f[1]) * sc.dx, d2 = -ar.f[2] * sc.dx;
-                    float t3[3], S = 0.0f, Sd = 0.0f;
+                    const float d1 = ((float)oy - ar.f[1]) * sc.dx;
+                    float t2[3], S = 0.0f, Sd = 0.0f;
 #pragma unroll
-                    for (int r = 0; r < 3; ++r)
-                        t3[r] = fmaf(Bq[r][2], d2, fmaf(Bq[r][1], d1, fmaf(Bq[r][0], d0, vb[r])));
+                    for (int r = 0; r < 3; ++r) t2[r] = fmaf(Bq[r][1], d1, fmaf(Bq[r][0], d0, vb[r]));
 #pragma unroll
                     for (int oz = 0; oz < 3; ++oz) {
                         const float4 v4 = s_v[((lc[0] + ox) * kTileSide + (lc[1] + oy)) * kTileSide + lc[2] + oz];
-                        const float q = fmaf(v4.x, t3[0], fmaf(v4.y, t3[1], v4.z * t3[2]));
+                        const float d2 = ((float)oz - ar.f[2]) * sc.dx;
+                        const float q = fmaf(v4.x, fmaf(Bq[0][2], d2, t2[0]),
+                                             fmaf(v4.y, fmaf(Bq[1][2], d2, t2[1]), v4.z * fmaf(Bq[2][2], d2, t2[2])));
                         S = fmaf(q, ar.w[2][oz], S);
                         Sd = fmaf(q, dw[2][oz], Sd);
-#pragma unroll
-                        for (int r = 0; r < 3; ++r) t3[r] += tz[r];
                     }
                     s0 = fmaf(S, ar.w[1][oy], s0);
                     s1 = fmaf(S, dw[1][oy], s1);
@@ -307,11 +304,9 @@ __global__ void __launch_bounds__(kAdjThreads) k_p2g_adjoint(State A, Partition 
 #pragma unroll
             for (int k = 0; k < 3; ++k) bspline_dw(ar.f[k], dw[k]);
             // line by line along z, as in the G2P adjoint: per node the momentum m v + B d the particle
-            // sends there (advanced by B's last column) and q = g_m m + g_mv . momentum; per line the sums
+            // sends there (B's last column alone changes along the line) and q = g_m m + g_mv . momentum; per line the sums
             // of w_z g_mv, w_z d_z g_mv, q w_z and q w'_z
-            float G0[3] = {0.0f, 0.0f, 0.0f}, Bb[3][3] = {{0.0f}}, gx[3] = {0.0f, 0.0f, 0.0f}, tz[3];
-#pragma unroll
-            for (int r = 0; r < 3; ++r) tz[r] = Bm[r][2] * sc.dx;
+            float G0[3] = {0.0f, 0.0f, 0.0f}, Bb[3][3] = {{0.0f}}, gx[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll 1
             for (int ox = 0; ox < 3; ++ox) {
                 const float wx = pick3(ar.w[0], ox), dwx = pick3(dw[0], ox), d0 = ((float)ox - ar.f[0]) * sc.dx;
@@ -320,22 +315,20 @@ __global__ void __launch_bounds__(kAdjThreads) k_p2g_adjoint(State A, Partition 
 #pragma unroll
                 for (int oy = 0; oy < 3; ++oy) {
                     const float d1 = ((float)oy - ar.f[1]) * sc.dx, wy = ar.w[1][oy];
-                    float t3[3], l0[3] = {0.0f, 0.0f, 0.0f}, lz[3] = {0.0f, 0.0f, 0.0f}, S = 0.0f, Sd = 0.0f;
+                    float t2[3], l0[3] = {0.0f, 0.0f, 0.0f}, lz[3] = {0.0f, 0.0f, 0.0f}, S = 0.0f, Sd = 0.0f;
 #pragma unroll
-                    for (int r = 0; r < 3; ++r)
-                        t3[r] = fmaf(Bm[r][2], -ar.f[2] * sc.dx, fmaf(Bm[r][1], d1, fmaf(Bm[r][0], d0, m * vp[r])));
+                    for (int r = 0; r < 3; ++r) t2[r] = fmaf(Bm[r][1], d1, fmaf(Bm[r][0], d0, m * vp[r]));
 #pragma unroll
                     for (int oz = 0; oz < 3; ++oz) {
                         const float4 g4 = s_g[((lc[0] + ox) * kTileSide + (lc[1] + oy)) * kTileSide + lc[2] + oz];
                         const float mvb[3] = {g4.y, g4.z, g4.w};
-                        const float wz = ar.w[2][oz], wdz = wz * (((float)oz - ar.f[2]) * sc.dx);
+                        const float d2 = ((float)oz - ar.f[2]) * sc.dx, wz = ar.w[2][oz], wdz = wz * d2;
                         float q = g4.x * m;
 #pragma unroll
                         for (int r = 0; r < 3; ++r) {
-                            q = fmaf(mvb[r], t3[r], q);
+                            q = fmaf(mvb[r], fmaf(Bm[r][2], d2, t2[r]), q);
                             l0[r] = fmaf(wz, mvb[r], l0[r]);
                             lz[r] = fmaf(wdz, mvb[r], lz[r]);
-                            t3[r] += tz[r];
                         }
                         S = fmaf(q, wz, S);
                         Sd = fmaf(q, dw[2][oz], Sd);
