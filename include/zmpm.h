@@ -250,6 +250,8 @@ ZMPM_API int32_t zmpm_create_scenes(zmpm_ctx **out, const zmpm_scene *scenes, in
 ZMPM_API int32_t zmpm_num_scenes(const zmpm_ctx *ctx);
 ZMPM_API int32_t zmpm_destroy(zmpm_ctx *ctx);
 ZMPM_API const char *zmpm_last_error(void);
+/* Later calls enqueue on hip_stream.  It neither waits for the work on the old stream nor orders the two:
+ * calls that use the same data (the resident state, a sort's buffers) are ordered by the caller. */
 ZMPM_API int32_t zmpm_set_stream(zmpm_ctx *ctx, void *hip_stream);
 ZMPM_API int32_t zmpm_sync(zmpm_ctx *ctx); /* synchronising; reports deferred device errors (ZMPM_ERR_DOMAIN) */
 
@@ -464,6 +466,10 @@ ZMPM_API int32_t zmpm_key_bits(const zmpm_ctx *ctx);
  * of src permuted into dst in code order (dst particle k = src particle ordered_to_original[k]).
  * Device pointers on the context's device; dst must not alias src; codes (optional) receives
  * the sorted codes.  n at most the context capacity (the sort uses the context's buffers).
+ * Asynchronous.  It shares the sort's buffers with imports, zmpm_sort_keys and the next reordering, and
+ * nothing with the resident state: substeps, graph replays and exports on another stream may run at the
+ * same time.  (From 65,536 particles on, a context with resident particles keeps 128 bytes of device
+ * memory per particle of its capacity for it from the first such call on, if there is that much.)
  * The reference's element ordering (IncludeElement) belongs to mesh primitives, not particles. */
 ZMPM_API int32_t zmpm_order_by_morton_code(zmpm_ctx *ctx, int32_t layout, int32_t nch, int64_t n, const float *src,
                                            float *dst, int32_t x_chn, const float bv_min[3], const float bv_max[3],

@@ -3785,11 +3785,14 @@ void launch_morton_codes(int32_t layout, int32_t nch, int64_t n, const float *sr
                        lo[1], lo[2], ext[0], ext[1], ext[2], codes);
 }
 
+bool permutes_by_records(int32_t layout, int32_t nch, int64_t n) {
+    return nch <= kRec && layout != ZMPM_LAYOUT_AOS && n >= kStageMin;
+}
+
 void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float *src, float *dst,
                              const uint32_t *order, float *rec, uint32_t *staged, hipStream_t s) {
     if (n <= 0) return;
-    const bool staging = rec && nch <= kRec && layout != ZMPM_LAYOUT_AOS && n >= kStageMin;
-    if (staging) {
+    if (rec) {
         launch_order_sample(order, kMortonLines, State{}, n, staged, s);
         hipLaunchKernelGGL(k_channels_to_rec, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, layout, nch, n, src, rec,
                            (const uint32_t *)staged);
@@ -3797,7 +3800,7 @@ void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float
                            (const float *)rec, dst, order, (const uint32_t *)staged);
     }
     hipLaunchKernelGGL(k_permute_channels, dim3(grid_for(n, 8192)), dim3(kThreads), 0, s, layout, nch, n, src, dst,
-                       order, staging ? (const uint32_t *)staged : nullptr);
+                       order, rec ? (const uint32_t *)staged : nullptr);
 }
 
 void launch_g2p_update(bool scatter, State A, State Bst, Partition P, Partition Pn, Lattice L, const float *grid,

@@ -128,9 +128,31 @@ struct zmpm_ctx {
     int grid_part = 0;  // the partition the grid values belong to
 
     uint32_t *keys = nullptr, *skeys = nullptr, *perm = nullptr;
-    uint32_t *staged = nullptr;  // k_order_sample's word
-    // between calls st[cur ^ 1] holds nothing: the records of an export or a reordering lie there
+    uint32_t *staged = nullptr;  // k_order_sample's words: of import and export, of the Morton reordering
+    // An export reads the state, so it comes after what wrote it and before what writes it again: its
+    // records lie in st[cur ^ 1], which holds nothing between calls.
     float *records() const { return st[cur ^ 1].ch; }
+    // The Morton reordering takes part in no such order: after zmpm_set_stream, or beside a replayed graph,
+    // it may run at once with substeps, so while particles are resident it has records of its own (128 bytes
+    // a particle of the capacity, made on first use; without the memory it permutes directly).
+    float *morton_rec = nullptr;
+    float *morton_records() {
+        if (n == 0) return records();  // no state: a later import shares the sort's buffers with this call anyway
+        if (!morton_rec && cap >= kStageMin) {
+            void *p = nullptr;
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // another thread may be capturing
+            HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+            const hipError_t err = hipMalloc(&p, sizeof(float) * 32 * (size_t)cap);
+            HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+            if (err != hipSuccess) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
+            allocations.push_back(p);
+            morton_rec = (float *)p;
+        }
+        return morton_rec;
+    }
     void *sort_scratch = nullptr;
     Binning bin{};
     float *tiles = nullptr, *grid = nullptr;
@@ -466,7 +488,7 @@ zmpm_ctx *create_context(const zmpm_scene *scenes, int32_t nscenes, int64_t capa
         c->keys = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->skeys = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->perm = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
-        c->staged = (uint32_t *)c->alloc(sizeof(uint32_t));
+        c->staged = (uint32_t *)c->alloc(2 * sizeof(uint32_t));
         c->sort_scratch = c->alloc(radix_scratch_bytes(cap));
         c->tiles = (float *)c->alloc(sizeof(float) * 4 * kTileNodes * parts_cap);
         c->tiles_blocks = parts_cap;
@@ -1740,16 +1762,17 @@ int32_t zmpm_order_by_morton_code(zmpm_ctx *ctx, int32_t layout, int32_t nch, in
         radix_sort_pairs(ctx->keys, nullptr, n, 0, 30, codes ? codes : ctx->skeys,
                          reinterpret_cast<uint32_t *>(ordered_to_original),
                          reinterpret_cast<uint32_t *>(original_to_ordered), ctx->sort_scratch, s);
-        // a captured launch may run when st[cur ^ 1] holds the state: it permutes directly
+        // captured, it permutes directly: when the graph runs is not known here
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        bool free_buffer = true;
+        bool eager = true;
         if (hipStreamIsCapturing(s, &capture) != hipSuccess) {
             (void)hipGetLastError();
-            free_buffer = false;
+            eager = false;
         }
-        free_buffer = free_buffer && capture == hipStreamCaptureStatusNone;
-        launch_permute_channels(layout, nch, n, src, dst, reinterpret_cast<const uint32_t *>(ordered_to_original),
-                                free_buffer ? ctx->records() : nullptr, ctx->staged, s);
+        eager = eager && capture == hipStreamCaptureStatusNone;
+        float *rec = eager && permutes_by_records(layout, nch, n) ? ctx->morton_records() : nullptr;
+        launch_permute_channels(layout, nch, n, src, dst, reinterpret_cast<const uint32_t *>(ordered_to_original), rec,
+                                ctx->staged + 1, s);
         HIP_CHECK(hipGetLastError());
     });
 }

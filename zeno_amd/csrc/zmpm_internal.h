@@ -372,7 +372,9 @@ void launch_particle_beta(State A, int64_t n, Lattice L, const DevMaterial *mats
 // permutation of every channel of src into dst by order (dst[k] = src[order[k]]).
 void launch_morton_codes(int32_t layout, int32_t nch, int64_t n, const float *src, int32_t x_chn, const float lo[3],
                          const float ext[3], uint32_t *codes, hipStream_t s);
-// rec: scratch of 32 floats per particle for the way through records (null: directly), staged: one word
+// rec: scratch of 32 floats per particle for the way through records (null: directly; given only where
+// permutes_by_records), staged: one word
+bool permutes_by_records(int32_t layout, int32_t nch, int64_t n);
 void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float *src, float *dst,
                              const uint32_t *order, float *rec, uint32_t *staged, hipStream_t s);
 
