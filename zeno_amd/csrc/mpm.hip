@@ -3202,12 +3202,16 @@ __global__ void __launch_bounds__(kThreads) k_export(State src, int64_t n_res, z
 
 // The same through records: resident particles -> records at their caller index -> the views.
 // want: the kAux* channels that a view asks for.
+// A loaded state may hold caller indices of n and more (it was saved when there were more particles): those
+// have no record, and then some entries of the views have no particle, so *staged is taken back and the
+// direct export does the work (it leaves such entries as they are).
 __global__ void __launch_bounds__(kThreads) k_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux,
-                                                            int want, float *rec, const uint32_t *staged) {
+                                                            int want, float *rec, uint32_t *staged) {
     __shared__ float s_rec[kRecWaves][64 * kRecPitch];
     if (*staged == 0u) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    bool beyond = false;
     for (int64_t k0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; k0 < n; k0 += (int64_t)gridDim.x * kThreads) {
         const uint32_t k = (uint32_t)min(k0 + lane, n - 1);
         const uint32_t mw = chan_u(src.ch, k, kChMat);
@@ -3232,8 +3236,11 @@ __global__ void __launch_bounds__(kThreads) k_export_to_rec(State src, int64_t n
                 r[kRecVol] = (aux & kAuxMass) ? chan(src.ch, k, kChVol) : mt.vol;
             }
         }
-        rec_put(s_rec[w], r, rec, k0 + lane < n ? chan_u(src.ch, k, kChPid) : kNoRec);
+        const uint32_t pid = chan_u(src.ch, k, kChPid);
+        beyond |= pid >= (uint32_t)n;
+        rec_put(s_rec[w], r, rec, k0 + lane < n && pid < (uint32_t)n ? pid : kNoRec);
     }
+    if (beyond) __hip_atomic_store(staged, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Records off .. off + v.n - 1 to the view (which asks for no fiber).
@@ -3939,7 +3946,7 @@ void launch_export(State src, int64_t n_res, const void *view, int64_t off, cons
 }
 
 void launch_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux, int want, float *rec,
-                          const uint32_t *staged, hipStream_t s) {
+                          uint32_t *staged, hipStream_t s) {
     hipLaunchKernelGGL(k_export_to_rec, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, src, n, mats, aux, want, rec,
                        staged);
 }

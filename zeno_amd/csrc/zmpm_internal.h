@@ -331,9 +331,9 @@ void launch_order_sample(const uint32_t *perm, uint32_t lines, State A, int64_t 
 // With staged, only one of launch_export and launch_export_to_rec + launch_rec_to_view does the work.
 void launch_export(State src, int64_t n_res, const void *view, int64_t off, const DevMaterial *mats, int aux,
                    const uint32_t *staged, hipStream_t s);
-// want: the kAux* channels to put into the records
+// want: the kAux* channels to put into the records; *staged = 0 if a particle's caller index is not below n
 void launch_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux, int want, float *rec,
-                          const uint32_t *staged, hipStream_t s);
+                          uint32_t *staged, hipStream_t s);
 void launch_rec_to_view(const float *rec, const void *view, int64_t off, const uint32_t *staged, hipStream_t s);
 // Particle volume dx^3 / (particles in the cell) and mass rho vol into caller buffers
 // (one channel each, ZMPM_LAYOUT_*) at the caller particle index; cnt: scratch of 64
