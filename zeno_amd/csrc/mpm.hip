@@ -168,11 +168,11 @@ __device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
 // particles has ceil(d / 2^L.part_shift) - 1 of them), so every block gets the number of
 // extra parts before it and every extra part its block and first particle.
 // The launch is a chain of dependent latencies (tile, entries, scan, look-back, entries), so the loads
-// of one step go out together, the scans are DPP adds and a lattice of at most 64 tiles takes them by
-// workgroup number.  1,331 entries: 8.1 -> 3.6 us, 42,875: 9.7 -> 4.7, 8 scenes: 11.7 -> 5.4, 300,763:
-// 12.2 -> 10.8, 256 scenes of 6.4 million (a tile finds its scene with the whole wave): 94 -> 60.
-// Tiles by workgroup number: the 64 workgroups that may wait never fill the chip (2,048 places), so
-// the one they wait for always gets a place; more tiles take a ticket.
+// of one step go out together and the scans are DPP adds.  1,331 entries: 8.1 -> 3.9 us, 42,875: 9.7 ->
+// 5.4, 8 scenes: 11.7 -> 6.0, 300,763: 12.2 -> 10.9, 256 scenes of 6.4 million (a tile finds its scene
+// with the whole wave): 94 -> 60.
+// A tile is taken by ticket, so the tiles it waits for have started, whatever else holds the chip's places.
+// (By workgroup number 0.4 us less, but a tile may then spin on one that waits for another stream's kernel.)
 __device__ __forceinline__ uint32_t extra_parts(uint32_t d, uint32_t shift) { return d == 0u ? 0u : (d - 1u) >> shift; }
 
 template <bool SMALL>
@@ -186,8 +186,8 @@ __global__ void __launch_bounds__(kScanThreads) k_lattice_scan(Lattice L, Partit
     // particle-block count in the low kPBlkBits bits (blocks <= capacity < 2^27), particles above
     constexpr uint64_t kBlkMask = (1ull << kPBlkBits) - 1;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t tile = blockIdx.x;
-    if (!SMALL && B.scan_tiles > kSmallScanTiles) {
+    uint32_t tile = 0u;
+    if (B.scan_tiles > 1) {
         if (threadIdx.x == 0) s_tile = atomicAdd(B.scan_p.tile_ctr, 1u);
         __syncthreads();
         tile = s_tile;
