@@ -2881,8 +2881,11 @@ __global__ void __launch_bounds__(kThreads) k_import(State dst, zmpm_particles v
 // into records, coalesced on both sides through LDS; the permuted side moves whole lines.  Export of
 // 4.9 million particles of 256 scenes: 1,936 -> 238 + 261 us, at 5 TB/s; import and permutation of a
 // shuffled 613,057: 48 + 240 -> 35 + 27 us.  It doubles the bytes, so an order that is local (runs of
-// a wave's 64 entries in few lines) keeps the direct kernels.  k_order_sample decides on the device,
-// without a synchronisation: both kinds are launched and one returns at once.
+// a wave's 64 entries in few lines) keeps the direct kernels.  For an import and a reordering
+// k_order_sample decides on the device, without a synchronisation: both kinds are launched and one returns
+// at once.  An export goes by the order that the last import or export read back with its status, and
+// launches one kind (three objects of 66,001, 200,003 and 700,001 particles in the cells' order: 70 -> 33,
+// 64 -> 39, 85 -> 66 us a call).
 constexpr int kRec = 32;
 constexpr int kRecPitch = 36;  // floats of a record's row in LDS: 16-byte rows on distinct banks
 constexpr int kRecWaves = kThreads / 64;
@@ -2932,16 +2935,16 @@ __device__ __forceinline__ void rec_get(float *s, float (&v)[kRec], const float 
     wave_lds_order();
 }
 
-// *staged = the order (perm, or the caller indices of the resident particles) is far from the
+// Whether an order (perm, or the caller indices of the resident particles) is far from the
 // memory's: 64 runs of 64 entries, evenly over the n >= 64, hold more than `lines` different
 // lines of 32 entries each on average (neighbours compared, so a line met again counts again); for an
-// export 10, and 16 for J-fluid particles, which move 17 channels in place of 25.
+// export 10, and 16 for J-fluid particles, which move 17 channels in place of 25.  By one workgroup of
+// 1,024; thread 0 has the result.
 // 2,000,000 solid particles shuffled within windows of 1, 64, 256, 4,096 and all entries hold 7, 10,
 // 25, 47 and 64 lines: an export takes 184, 218, 369, 638 and 972 us directly, 205 through records; an
 // import with its sort 319, 347, 417, 522 and 1,057, against 385.  At 600,000 the export: 63, 82, 116,
 // 159 and 203, against 71.  The dam of 4.2 million, 93 % fluid, 12 to 16 lines: 250 directly, 353.
-__global__ void __launch_bounds__(1024) k_order_sample(const uint32_t *perm, uint32_t lines, const float *ch,
-                                                       int64_t n, uint32_t *staged) {
+__device__ __forceinline__ bool order_sample(const uint32_t *perm, uint32_t lines, const float *ch, int64_t n) {
     __shared__ uint32_t s_lines[16], s_fluid[16];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     uint32_t found = 0, fluid = 0;
@@ -2958,14 +2961,20 @@ __global__ void __launch_bounds__(1024) k_order_sample(const uint32_t *perm, uin
         s_fluid[w] = fluid;
     }
     __syncthreads();
+    uint32_t total = 0, nf = 0;
     if (threadIdx.x == 0) {
-        uint32_t total = 0, nf = 0;
         for (int q = 0; q < 16; ++q) {
             total += s_lines[q];
             nf += s_fluid[q];
         }
-        *staged = total * 64u > (perm ? lines * 4096u : 10u * 4096u + 6u * nf) ? 1u : 0u;
     }
+    return total * 64u > (perm ? lines * 4096u : 10u * 4096u + 6u * nf);
+}
+
+__global__ void __launch_bounds__(1024) k_order_sample(const uint32_t *perm, uint32_t lines, int64_t n,
+                                                       uint32_t *staged) {
+    const bool far = order_sample(perm, lines, nullptr, n);
+    if (threadIdx.x == 0) *staged = far ? 1u : 0u;
 }
 
 // Keys of the view's particles, as k_bin_keys makes them from the resident ones.
@@ -3137,8 +3146,7 @@ __global__ void __launch_bounds__(kThreads) k_rec_to_channels(int32_t layout, in
 // as their initial values (the material's flip_beta, logJp -0.04).
 // Resident particles of caller index off .. off + v.n - 1 go to the view's entries 0 .. v.n - 1.
 __global__ void __launch_bounds__(kThreads) k_export(State src, int64_t n_res, zmpm_particles v, int64_t off,
-                                                     const DevMaterial *mats, int aux, const uint32_t *staged) {
-    if (staged && *staged != 0u) return;
+                                                     const DevMaterial *mats, int aux) {
     const int64_t n = v.n;
     for (int64_t k = blockIdx.x * (int64_t)kThreads + threadIdx.x; k < n_res; k += (int64_t)gridDim.x * kThreads) {
         const int64_t i = (int64_t)chan_u(src.ch, (uint32_t)k, kChPid) - off;
@@ -3203,15 +3211,14 @@ __global__ void __launch_bounds__(kThreads) k_export(State src, int64_t n_res, z
 // The same through records: resident particles -> records at their caller index -> the views.
 // want: the kAux* channels that a view asks for.
 // A loaded state may hold caller indices of n and more (it was saved when there were more particles): those
-// have no record, and then some entries of the views have no particle, so *staged is taken back and the
+// have no record, and then some entries of the views have no particle, so *beyond is set and the
 // direct export does the work (it leaves such entries as they are).
 __global__ void __launch_bounds__(kThreads) k_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux,
-                                                            int want, float *rec, uint32_t *staged) {
+                                                            int want, float *rec, uint32_t *beyond) {
     __shared__ float s_rec[kRecWaves][64 * kRecPitch];
-    if (*staged == 0u) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    bool beyond = false;
+    bool out = false;
     for (int64_t k0 = ((int64_t)blockIdx.x * kRecWaves + w) * 64; k0 < n; k0 += (int64_t)gridDim.x * kThreads) {
         const uint32_t k = (uint32_t)min(k0 + lane, n - 1);
         const uint32_t mw = chan_u(src.ch, k, kChMat);
@@ -3237,17 +3244,17 @@ __global__ void __launch_bounds__(kThreads) k_export_to_rec(State src, int64_t n
             }
         }
         const uint32_t pid = chan_u(src.ch, k, kChPid);
-        beyond |= pid >= (uint32_t)n;
+        out |= pid >= (uint32_t)n;
         rec_put(s_rec[w], r, rec, k0 + lane < n && pid < (uint32_t)n ? pid : kNoRec);
     }
-    if (beyond) __hip_atomic_store(staged, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (out) __hip_atomic_store(beyond, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Records off .. off + v.n - 1 to the view (which asks for no fiber).
 __global__ void __launch_bounds__(kThreads) k_rec_to_view(const float *rec, zmpm_particles v, int64_t off,
-                                                          const uint32_t *staged) {
+                                                          const uint32_t *beyond) {
     __shared__ float s_rec[kRecWaves][64 * kRecPitch];
-    if (*staged == 0u) return;
+    if (*beyond != 0u) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t n = v.n;
@@ -3477,15 +3484,19 @@ __global__ void __launch_bounds__(kThreads) k_cell_volume(State A, int64_t n, Pa
     }
 }
 
+// Words that the host waits for (launch_read_back).
+__global__ void __launch_bounds__(1024) k_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb,
+                                                    const float *ch, int64_t n, uint32_t *host) {
+    for (int32_t i = threadIdx.x; i < na + nb; i += blockDim.x) host[i] = i < na ? a[i] : b[i - na];
+    if (!ch) return;
+    const bool far = order_sample(nullptr, 0u, ch, n);
+    if (threadIdx.x == 0) host[na + nb] = far ? 1u : 0u;
+}
+
 // Per-scene max |v|^2 from the per-grid-block maxima (out zeroed by the caller):
 // one atomic max on the float bits per wave whose blocks share a scene, per lane
 // otherwise.  Non-negative floats order as their bits, and max is order
 // independent, so the result is deterministic.
-__global__ void __launch_bounds__(kThreads) k_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb,
-                                                        uint32_t *host) {
-    for (int32_t i = threadIdx.x; i < na + nb; i += kThreads) host[i] = i < na ? a[i] : b[i - na];
-}
-
 __global__ void __launch_bounds__(kThreads) k_reduce_vmax(const float *gvmax, const uint32_t *gblk_scene,
                                                           const uint32_t *counts, uint32_t *out) {
     const uint32_t ng = counts[1];
@@ -3715,8 +3726,10 @@ void launch_grid(int mode, Partition P, Lattice L, const float *tiles, float *gr
                        grid, gvmax, out ? out : grid, vclear, nclear);
 }
 
-void launch_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb, uint32_t *host, hipStream_t s) {
-    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(kThreads), 0, s, a, na, b, nb, host);
+void launch_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb, State A, int64_t n, uint32_t *host,
+                      hipStream_t s) {
+    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(A.ch ? 1024 : kThreads), 0, s, a, na, b, nb, (const float *)A.ch, n,
+                       host);
 }
 
 void launch_reduce_vmax(const float *gvmax, Partition P, int64_t max_blocks, uint32_t *out, hipStream_t s) {
@@ -3800,7 +3813,7 @@ void launch_permute_channels(int32_t layout, int32_t nch, int64_t n, const float
                              const uint32_t *order, float *rec, uint32_t *staged, hipStream_t s) {
     if (n <= 0) return;
     if (rec) {
-        launch_order_sample(order, kMortonLines, State{}, n, staged, s);
+        launch_order_sample(order, kMortonLines, n, staged, s);
         hipLaunchKernelGGL(k_channels_to_rec, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, layout, nch, n, src, rec,
                            (const uint32_t *)staged);
         hipLaunchKernelGGL(k_rec_to_channels, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, layout, nch, n,
@@ -3857,8 +3870,8 @@ void launch_import(State dst, const void *view, int64_t off, const DevMaterial *
     hipLaunchKernelGGL(k_import, dim3(grid_for(v.n, 8192)), dim3(kThreads), 0, s, dst, v, off, mats, nmat, st);
 }
 
-void launch_order_sample(const uint32_t *perm, uint32_t lines, State A, int64_t n, uint32_t *staged, hipStream_t s) {
-    hipLaunchKernelGGL(k_order_sample, dim3(1), dim3(1024), 0, s, perm, lines, (const float *)A.ch, n, staged);
+void launch_order_sample(const uint32_t *perm, uint32_t lines, int64_t n, uint32_t *staged, hipStream_t s) {
+    hipLaunchKernelGGL(k_order_sample, dim3(1), dim3(1024), 0, s, perm, lines, n, staged);
 }
 
 void launch_view_keys(const void *view, int64_t off, const DevMaterial *mats, int32_t nmat, Lattice L, uint32_t *keys,
@@ -3938,23 +3951,22 @@ void launch_particle_volume(State A, int64_t n, Partition P, Lattice L, const De
 }
 
 void launch_export(State src, int64_t n_res, const void *view, int64_t off, const DevMaterial *mats, int aux,
-                   const uint32_t *staged, hipStream_t s) {
+                   hipStream_t s) {
     const zmpm_particles v = *(const zmpm_particles *)view;
     if (v.n <= 0 || n_res <= 0) return;
-    hipLaunchKernelGGL(k_export, dim3(grid_for(n_res, 8192)), dim3(kThreads), 0, s, src, n_res, v, off, mats, aux,
-                       staged);
+    hipLaunchKernelGGL(k_export, dim3(grid_for(n_res, 8192)), dim3(kThreads), 0, s, src, n_res, v, off, mats, aux);
 }
 
 void launch_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux, int want, float *rec,
-                          uint32_t *staged, hipStream_t s) {
+                          uint32_t *beyond, hipStream_t s) {
     hipLaunchKernelGGL(k_export_to_rec, dim3(grid_for(n, 4096)), dim3(kThreads), 0, s, src, n, mats, aux, want, rec,
-                       staged);
+                       beyond);
 }
 
-void launch_rec_to_view(const float *rec, const void *view, int64_t off, const uint32_t *staged, hipStream_t s) {
+void launch_rec_to_view(const float *rec, const void *view, int64_t off, const uint32_t *beyond, hipStream_t s) {
     const zmpm_particles v = *(const zmpm_particles *)view;
     if (v.n <= 0) return;
-    hipLaunchKernelGGL(k_rec_to_view, dim3(grid_for(v.n, 4096)), dim3(kThreads), 0, s, rec, v, off, staged);
+    hipLaunchKernelGGL(k_rec_to_view, dim3(grid_for(v.n, 4096)), dim3(kThreads), 0, s, rec, v, off, beyond);
 }
 
 }  // namespace zmpm

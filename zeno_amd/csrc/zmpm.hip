@@ -128,7 +128,11 @@ struct zmpm_ctx {
     int grid_part = 0;  // the partition the grid values belong to
 
     uint32_t *keys = nullptr, *skeys = nullptr, *perm = nullptr;
-    uint32_t *staged = nullptr;  // k_order_sample's words: of import and export, of the Morton reordering
+    uint32_t *staged = nullptr;  // k_order_sample's words: of the import, of the Morton reordering
+    uint32_t *beyond = nullptr;  // k_export_to_rec's word; zero between calls
+    // the resident particles' order is far from their callers', as the last import or export found it: what
+    // the next export goes by (either way gives the same)
+    bool order_far = false;
     // An export reads the state, so it comes after what wrote it and before what writes it again: its
     // records lie in st[cur ^ 1], which holds nothing between calls.
     float *records() const { return st[cur ^ 1].ch; }
@@ -272,15 +276,16 @@ void check_ctx(const zmpm_ctx *c) {
     if (!c) throw ZmpmError(ZMPM_ERR_ARG, "null context");
 }
 
-// The status words and, with vmax, the scenes' MaxVelSqr words after them into host memory
-// (synchronising): a kernel writes them there and the stream is waited for.  (A copy to ordinary host
-// memory goes through the runtime's staging and a wait of its own: 20 us with an idle stream, this way 12.)
-const uint32_t *read_back(zmpm_ctx *c, bool vmax) {
+// The status words, then nmore others and, with order, order_far anew, into host memory (synchronising): a
+// kernel writes them there and the stream is waited for.  (A copy to ordinary host memory goes through
+// the runtime's staging and a wait of its own: 20 us with an idle stream, this way 12.)
+const uint32_t *read_back(zmpm_ctx *c, const uint32_t *more = nullptr, int32_t nmore = 0, bool order = false) {
     constexpr int32_t words = sizeof(DevStatus) / sizeof(uint32_t);
-    launch_read_back(reinterpret_cast<const uint32_t *>(c->status), words, c->vmax, vmax ? c->L.nscenes : 0,
-                     c->host_back_dev, c->stream);
+    launch_read_back(reinterpret_cast<const uint32_t *>(c->status), words, more, nmore,
+                     order ? c->st[c->cur] : State{}, c->n, c->host_back_dev, c->stream);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(c->stream));
+    if (order) c->order_far = c->host_back[words + nmore] != 0u;
     return c->host_back + words;
 }
 
@@ -298,7 +303,7 @@ void throw_status(const zmpm_ctx *c) {
 }
 
 void check_status(zmpm_ctx *c) {
-    read_back(c, false);
+    read_back(c);
     throw_status(c);
 }
 
@@ -318,7 +323,7 @@ void import_sorted(zmpm_ctx *c, const zmpm_particles *views, int32_t nviews, boo
     sort_by_block(c);
     float *rec = records ? c->st[c->cur].ch : nullptr;
     uint32_t *staged = records && nviews == 1 ? c->staged : nullptr;
-    if (staged) launch_order_sample(c->perm, kImportLines, State{}, c->n, staged, s);
+    if (staged) launch_order_sample(c->perm, kImportLines, c->n, staged, s);
     off = 0;
     for (int k = 0; rec && k < nviews; off += views[k++].n)
         launch_view_to_rec(&views[k], off, c->mats, c->nmat, rec, staged, s);
@@ -482,13 +487,15 @@ zmpm_ctx *create_context(const zmpm_scene *scenes, int32_t nscenes, int64_t capa
         HIP_CHECK(hipHostMalloc((void **)&c->host_counts, 4 * sizeof(uint32_t), hipHostMallocMapped));
         std::memset(c->host_counts, 0, 4 * sizeof(uint32_t));
         HIP_CHECK(hipHostGetDevicePointer((void **)&B.host_counts, c->host_counts, 0));
-        HIP_CHECK(hipHostMalloc((void **)&c->host_back, sizeof(DevStatus) + sizeof(uint32_t) * nscenes,
+        HIP_CHECK(hipHostMalloc((void **)&c->host_back, sizeof(DevStatus) + sizeof(uint32_t) * (nscenes + 1),
                                 hipHostMallocMapped));
         HIP_CHECK(hipHostGetDevicePointer((void **)&c->host_back_dev, c->host_back, 0));
         c->keys = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->skeys = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->perm = (uint32_t *)c->alloc(sizeof(uint32_t) * cap);
         c->staged = (uint32_t *)c->alloc(2 * sizeof(uint32_t));
+        c->beyond = (uint32_t *)c->alloc(sizeof(uint32_t));
+        HIP_CHECK(hipMemset(c->beyond, 0, sizeof(uint32_t)));
         c->sort_scratch = c->alloc(radix_scratch_bytes(cap));
         c->tiles = (float *)c->alloc(sizeof(float) * 4 * kTileNodes * parts_cap);
         c->tiles_blocks = parts_cap;
@@ -722,7 +729,8 @@ void import_views(zmpm_ctx *ctx, const zmpm_particles *views, int32_t nviews) {
     }
     HIP_CHECK(hipGetLastError());
     full_partition(ctx, 0, sorted);
-    check_status(ctx);
+    read_back(ctx, nullptr, 0, total >= kStageMin);
+    throw_status(ctx);
 }
 
 void export_views(zmpm_ctx *ctx, const zmpm_particles *views, int32_t nviews) {
@@ -734,19 +742,25 @@ void export_views(zmpm_ctx *ctx, const zmpm_particles *views, int32_t nviews) {
     for (int k = 0; k < nviews; ++k)
         want |= (views[k].beta ? kAuxBeta : 0) | (views[k].logJp ? kAuxLogJp : 0) | (views[k].mu ? kAuxLame : 0) |
                 (views[k].a ? kAuxFiber : 0) | (views[k].m ? kAuxMass : 0);
-    uint32_t *staged = ctx->n >= kStageMin && !(want & kAuxFiber) ? ctx->staged : nullptr;
-    if (staged) {
-        launch_order_sample(nullptr, 0, ctx->st[ctx->cur], ctx->n, staged, ctx->stream);
-        launch_export_to_rec(ctx->st[ctx->cur], ctx->n, ctx->mats, ctx->aux(), want, ctx->records(), staged,
+    bool records = ctx->n >= kStageMin && ctx->order_far && !(want & kAuxFiber);
+    if (records) {
+        launch_export_to_rec(ctx->st[ctx->cur], ctx->n, ctx->mats, ctx->aux(), want, ctx->records(), ctx->beyond,
                              ctx->stream);
+        int64_t off = 0;
+        for (int k = 0; k < nviews; off += views[k++].n)
+            launch_rec_to_view(ctx->records(), &views[k], off, ctx->beyond, ctx->stream);
+        if (*read_back(ctx, ctx->beyond, 1, true) != 0u) {
+            fill_u32(ctx->beyond, 0u, 1, ctx->stream);
+            records = false;
+        }
     }
-    int64_t off = 0;
-    for (int k = 0; k < nviews; off += views[k++].n) {
-        if (staged) launch_rec_to_view(ctx->records(), &views[k], off, staged, ctx->stream);
-        launch_export(ctx->st[ctx->cur], ctx->n, &views[k], off, ctx->mats, ctx->aux(), staged, ctx->stream);
+    if (!records) {
+        int64_t off = 0;
+        for (int k = 0; k < nviews; off += views[k++].n)
+            launch_export(ctx->st[ctx->cur], ctx->n, &views[k], off, ctx->mats, ctx->aux(), ctx->stream);
+        read_back(ctx, nullptr, 0, ctx->n >= kStageMin);
     }
-    HIP_CHECK(hipGetLastError());
-    check_status(ctx);
+    throw_status(ctx);
 }
 
 }  // namespace
@@ -1157,7 +1171,7 @@ int32_t zmpm_scene_max_vel_sqr(zmpm_ctx *ctx, float *out, int32_t nscenes) {
         ctx->set_device();
         const int k = std::min<int>(nscenes, ctx->L.nscenes);
         reduce_vmax(ctx);
-        const uint32_t *bits = read_back(ctx, true);
+        const uint32_t *bits = read_back(ctx, ctx->vmax, ctx->L.nscenes);
         for (int i = 0; i < k; ++i) std::memcpy(&out[i], &bits[i], sizeof(float));
         throw_status(ctx);
     });
@@ -1177,7 +1191,7 @@ int32_t zmpm_max_vel_sqr(zmpm_ctx *ctx, float *out) {
         if (!out) throw ZmpmError(ZMPM_ERR_ARG, "null output");
         ctx->set_device();
         reduce_vmax(ctx);
-        const uint32_t *bits = read_back(ctx, true);
+        const uint32_t *bits = read_back(ctx, ctx->vmax, ctx->L.nscenes);
         uint32_t mx = 0;  // non-negative floats order as their bits
         for (int32_t i = 0; i < ctx->L.nscenes; ++i) mx = std::max(mx, bits[i]);
         std::memcpy(out, &mx, sizeof(float));

@@ -265,8 +265,10 @@ void launch_grid(int mode, Partition P, Lattice L, const float *tiles, float *gr
                  int32_t nclear = 0);
 // out[scene] = max over the scene's grid blocks of gvmax, as float bits (out zeroed first)
 void launch_reduce_vmax(const float *gvmax, Partition P, int64_t max_blocks, uint32_t *out, hipStream_t s);
-// a[0 .. na), then b[0 .. nb), to host (device-mapped host memory)
-void launch_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb, uint32_t *host, hipStream_t s);
+// a[0 .. na), then b[0 .. nb), to host (device-mapped host memory), then, if A has channels, whether its
+// n >= 64 particles' order is far from their callers' (k_order_sample's test)
+void launch_read_back(const uint32_t *a, int32_t na, const uint32_t *b, int32_t nb, State A, int64_t n, uint32_t *host,
+                      hipStream_t s);
 // G2P pass 1 of the fused substep: direction of each particle's new block, per-block
 // direction counts, destination marks.  Also resets the lattice scan's state.
 // wg: threads per workgroup, 64 or 256 (one particle block per workgroup either way)
@@ -322,19 +324,20 @@ void launch_view_to_rec(const void *view, int64_t off, const DevMaterial *mats, 
                         const uint32_t *staged, hipStream_t s);
 void launch_import_sorted(State dst, const void *view, const float *rec, const uint32_t *perm, int64_t n,
                           const DevMaterial *mats, int32_t nmat, const uint32_t *staged, hipStream_t s);
-// *staged = whether perm (null: the resident particles' caller indices) is so far from memory order
-// that moving the particles through records is the faster way (n >= 64): more than `lines` lines a run
+// *staged = whether perm is so far from memory order that moving the particles through records is the
+// faster way (n >= 64): more than `lines` lines a run
 constexpr uint32_t kImportLines = 16, kMortonLines = 12;
-void launch_order_sample(const uint32_t *perm, uint32_t lines, State A, int64_t n, uint32_t *staged, hipStream_t s);
+void launch_order_sample(const uint32_t *perm, uint32_t lines, int64_t n, uint32_t *staged, hipStream_t s);
 // aux: the kAux* channels the resident state keeps (the others are exported as their initial values);
 // the resident particles of caller index off .. off + view->n - 1 go to the view's entries 0 .. n - 1.
-// With staged, only one of launch_export and launch_export_to_rec + launch_rec_to_view does the work.
+// launch_export does it directly, launch_export_to_rec and launch_rec_to_view through records.
 void launch_export(State src, int64_t n_res, const void *view, int64_t off, const DevMaterial *mats, int aux,
-                   const uint32_t *staged, hipStream_t s);
-// want: the kAux* channels to put into the records; *staged = 0 if a particle's caller index is not below n
+                   hipStream_t s);
+// want: the kAux* channels to put into the records.  *beyond = 1 if a particle's caller index is not below
+// n: launch_rec_to_view then does nothing, and launch_export has to do the work.
 void launch_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux, int want, float *rec,
-                          uint32_t *staged, hipStream_t s);
-void launch_rec_to_view(const float *rec, const void *view, int64_t off, const uint32_t *staged, hipStream_t s);
+                          uint32_t *beyond, hipStream_t s);
+void launch_rec_to_view(const float *rec, const void *view, int64_t off, const uint32_t *beyond, hipStream_t s);
 // Particle volume dx^3 / (particles in the cell) and mass rho vol into caller buffers
 // (one channel each, ZMPM_LAYOUT_*) at the caller particle index; cnt: scratch of 64
 // words per grid block.
