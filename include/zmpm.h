@@ -375,7 +375,8 @@ ZMPM_API int32_t zmpm_substeps(zmpm_ctx *ctx, const zmpm_step_params *params, in
 /* Time each candidate workgroup size of the two G2P kernels (64 or 256 threads per particle
  * block), P2G with and without the one-wave kernel for blocks of at most 64 particles, and (APIC)
  * the fused G2P / P2G pass, over nsteps substeps from the current state, keep the fastest, and
- * restore the state (no counterpart in the reference).  Results do not depend on the choice.
+ * restore the state (no counterpart in the reference).  Results do not depend on the choice, which holds
+ * until the next call; before the first, the number of block parts decides (also for 512 threads).
  * choice (optional, 3 entries) receives the G2P move size, the G2P update size (0 when the fused
  * pass won: it replaces G2P update, the stress and P2G kernels) and 1 if the one-wave P2G is on. */
 ZMPM_API int32_t zmpm_autotune(zmpm_ctx *ctx, const zmpm_step_params *params, int32_t nsteps, int32_t *choice);

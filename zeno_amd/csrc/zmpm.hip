@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../include/zmpm.h"
+#include "launch_rules.h"
 #include "zmpm_internal.h"
 
 using namespace zmpm;
@@ -74,34 +75,10 @@ struct zmpm_ctx {
         const volatile uint32_t *c = host_counts;
         return c && c[0] ? (int64_t)c[0] + c[2] : max_units();
     }
-    // Threads per workgroup (one part each) of the G2P kernels: as zmpm_autotune found, else by how
-    // many parts there are.  Few leave wave slots empty, so a part gets as many threads as pay; many
-    // fill the chip with one wave each, which waits at no barrier.
-    // Move, 180 parts of 363 particles: 12.4 us with 64 threads, 8.4 with 256, 8.2 with 512; 1,180 of
-    // 340: 15.1, 10.8, 16.9; 1,800 of 340: 16.5, 17.7, 24.2; 9,990 of 420: 46, 67, 114; 77,514 of 60:
-    // 165, 319, -.  Update, the same: 22.1, 12.4, 10.8; 27.8, 19.0, 21.7; 27.8, 25.5, 30.4; 127, 119,
-    // 153; 340, 506, -; about 400 parts: 24.9, 14.1, 13.0; 740: 26.5, 16.4, 18.4.
-    // FLIP transfers (the particles are all interpolated, twice the registers), move and update, 366
-    // parts: 27 and 34 with 64, 16 and 16 with 256, 15 and 19 with 512; 1,750: 37 and 44, 28 and 44, 34
-    // and 54; 5,800: 87 and 159, 68 and 144, 95 and 170.
-    int wg_move_tuned = 0, wg_update_tuned = 0;
-    bool many_small_parts() const { return parts_now() >= 1536 && n <= 96 * parts_now(); }
-    int wg_move() const {
-        if (wg_move_tuned) return wg_move_tuned;
-        return (flip_style() ? many_small_parts() : parts_now() >= 1536) ? 64 : 256;
-    }
-    int wg_update() const {
-        if (wg_update_tuned == 64 || (!wg_update_tuned && many_small_parts())) return 64;
-        return !flip_style() && parts_now() <= 512 ? 512 : 256;
-    }
-    // one-wave P2G for blocks of <= 64 particles, a launch of its own: as zmpm_autotune found, else
-    // where the chip is full of blocks that hold few particles.  (A launch that finds no such block
-    // still costs 13-18 us; on 77,514 blocks of 60 particles on average it gains 423 against 440 us.)
-    int p2g_sparse_tuned = -1;
-    bool p2g_sparse() const {
-        if (p2g_sparse_tuned >= 0) return p2g_sparse_tuned != 0;
-        return parts_now() >= 16384 && n <= 96 * parts_now();
-    }
+    int wg_move_tuned = 0, wg_update_tuned = 0, p2g_sparse_tuned = -1;  // zmpm_autotune's choice
+    int wg_move() const { return g2p_move_threads(parts_now(), n, flip_style(), wg_move_tuned); }
+    int wg_update() const { return g2p_update_threads(parts_now(), n, flip_style(), wg_update_tuned); }
+    bool p2g_sparse() const { return p2g_one_wave(parts_now(), n, p2g_sparse_tuned); }
     bool fuse = false;                   // APIC: the fused G2P / P2G pass (zmpm_autotune, zmpm_set_fused);
                                          // while on, every P2G of the context uses its chunk-flush grouping
     bool tiles_valid = false;            // fused pass: tiles hold the P2G of the current state and partition
