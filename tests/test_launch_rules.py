@@ -52,3 +52,10 @@ def test_untuned_sizes_exist(rules):
     for c, (move, update, wave) in zip(cases, rules(cases)):
         assert move in (64, 256) and update in ((64, 256) if c[2] else (64, 256, 512)) and wave in (0, 1)
         assert c[0] >= 1536 or (move, wave) == (256, 0)
+
+
+def test_one_wave_p2g_only_for_small_blocks(rules):
+    """Blocks of 60 particles on average, many of more than 64, are faster without it."""
+    assert [r[2] for r in rules([(77514, 77514 * k, 0, 0, 0, -1) for k in (20, 48, 49, 60)])] == [1, 1, 0, 0]
+    assert [r[2] for r in rules([(32767, 32767 * k, 0, 0, 0, -1) for k in (36, 37)])] == [1, 0]
+    assert [r[2] for r in rules([(p, p * 20, 0, 0, 0, -1) for p in (16383, 16384)])] == [0, 1]
