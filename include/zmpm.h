@@ -391,7 +391,9 @@ ZMPM_API int32_t zmpm_fused(const zmpm_ctx *ctx);
 
 /* Capture nsteps (even) fused substeps into a HIP graph on the context stream, replayed by
  * zmpm_graph_launch (no counterpart in the reference).  The state must not be re-imported or
- * re-partitioned between capture and launch; capturing again replaces the graph. */
+ * re-partitioned between capture and launch; capturing again replaces the graph.  The graph keeps the
+ * kernels and launch sizes chosen for the block counts at the capture: replays with any counts give the
+ * same results, and when the counts have grown several times over, capturing again is faster. */
 ZMPM_API int32_t zmpm_graph_capture(zmpm_ctx *ctx, const zmpm_step_params *params, int32_t nsteps);
 ZMPM_API int32_t zmpm_graph_launch(zmpm_ctx *ctx);
 

@@ -783,6 +783,15 @@ __device__ __forceinline__ void p2g_chunk_tail(float *s_pl, const uint8_t *s_tas
     p2g_tiles_out(acc, s_pl, s_task, tb, first);
 }
 
+// LDS of k_p2g.
+struct P2GShared {
+    float pl[kPL * kP2GChunk];
+    uint32_t wcnt[kP2GRounds * 3][64];
+    uint32_t cstart[65];
+    uint8_t task[3 * 64];  // phase B task p -> cell (x-offset p % 3)
+};
+static_assert(3 * kTileNodes * 4 <= kPL * kP2GChunk, "tiles alias the payload");
+
 // P2G (Transfer.cu:844-890) of one particle block per workgroup, into the block's
 // 6^3 tile.  A block's particles are staged in chunks of kP2GChunk; the
 // registers carry each lane's sums from one chunk to the next.
@@ -808,15 +817,7 @@ __device__ __forceinline__ void p2g_chunk_tail(float *s_pl, const uint8_t *s_tas
 // phases C and D on their own, p2g_chunk_tail); otherwise the registers carry each
 // task's sums from one chunk to the next and phases C and D run once per block.
 // The two agree bit for bit on blocks of at most kP2GChunk particles.
-struct P2GShared {
-    float pl[kPL * kP2GChunk];
-    uint32_t wcnt[kP2GRounds * 3][64];
-    uint32_t cstart[65];
-    uint8_t task[3 * 64];  // phase B task p -> cell (x-offset p % 3)
-};
-static_assert(3 * kTileNodes * 4 <= kPL * kP2GChunk, "tiles alias the payload");
-
-// The parts first, first + stride, ... of the partition.
+// p2g_parts: the parts first, first + stride, ... of the partition.
 template <int MODE, bool PP, bool FLUSH>
 __device__ __forceinline__ void p2g_parts(P2GShared &sh, uint32_t first, uint32_t stride, State A,
                                           const Partition &P, const Lattice &L, const DevMaterial *mats,
@@ -2995,7 +2996,7 @@ __global__ void __launch_bounds__(kThreads) k_view_keys(zmpm_particles v, int64_
 // View -> records at the caller index (the view carries no fiber).
 __global__ void __launch_bounds__(kThreads) k_view_to_rec(zmpm_particles v, int64_t off, const DevMaterial *mats,
                                                           int32_t nmat, float *rec, const uint32_t *staged) {
-    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    __shared__ alignas(16) float s_rec[kRecWaves][64 * kRecPitch];
     if (staged && *staged == 0u) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -3023,7 +3024,7 @@ template <bool DIRECT>
 __global__ void __launch_bounds__(kThreads) k_import_sorted(State dst, zmpm_particles v, const float *rec,
                                                             const uint32_t *perm, int64_t n, const DevMaterial *mats,
                                                             int32_t nmat, const uint32_t *staged) {
-    __shared__ float s_rec[DIRECT ? 1 : kRecWaves][64 * kRecPitch];
+    __shared__ alignas(16) float s_rec[DIRECT ? 1 : kRecWaves][64 * kRecPitch];
     if (staged && (*staged != 0u) == DIRECT) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -3112,7 +3113,7 @@ __global__ void __launch_bounds__(kThreads) k_permute_channels(int32_t layout, i
 
 __global__ void __launch_bounds__(kThreads) k_channels_to_rec(int32_t layout, int32_t nch, int64_t n, const float *src,
                                                               float *rec, const uint32_t *staged) {
-    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    __shared__ alignas(16) float s_rec[kRecWaves][64 * kRecPitch];
     if (*staged == 0u) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -3128,7 +3129,7 @@ __global__ void __launch_bounds__(kThreads) k_channels_to_rec(int32_t layout, in
 __global__ void __launch_bounds__(kThreads) k_rec_to_channels(int32_t layout, int32_t nch, int64_t n, const float *rec,
                                                               float *dst, const uint32_t *order,
                                                               const uint32_t *staged) {
-    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    __shared__ alignas(16) float s_rec[kRecWaves][64 * kRecPitch];
     if (*staged == 0u) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -3215,7 +3216,7 @@ __global__ void __launch_bounds__(kThreads) k_export(State src, int64_t n_res, z
 // direct export does the work (it leaves such entries as they are).
 __global__ void __launch_bounds__(kThreads) k_export_to_rec(State src, int64_t n, const DevMaterial *mats, int aux,
                                                             int want, float *rec, uint32_t *beyond) {
-    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    __shared__ alignas(16) float s_rec[kRecWaves][64 * kRecPitch];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     bool out = false;
@@ -3253,7 +3254,7 @@ __global__ void __launch_bounds__(kThreads) k_export_to_rec(State src, int64_t n
 // Records off .. off + v.n - 1 to the view (which asks for no fiber).
 __global__ void __launch_bounds__(kThreads) k_rec_to_view(const float *rec, zmpm_particles v, int64_t off,
                                                           const uint32_t *beyond) {
-    __shared__ float s_rec[kRecWaves][64 * kRecPitch];
+    __shared__ alignas(16) float s_rec[kRecWaves][64 * kRecPitch];
     if (*beyond != 0u) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

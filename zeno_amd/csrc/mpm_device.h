@@ -58,17 +58,6 @@ __device__ __forceinline__ SceneParams scene_params(const Lattice &L, uint32_t s
     return L.nscenes == 1 ? L.s0 : L.scenes[scene];
 }
 
-// Scene owning lattice entry l (binary search over the scenes' first entries).
-__device__ __forceinline__ int scene_of(const Lattice &L, int64_t l) {
-    int lo = 0, hi = L.nscenes - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (L.scenes[mid].lat_off <= l) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 // Quadratic B-spline weights of one axis from the fractional position f
 // (the same expressions as make_arena).
 __device__ __forceinline__ void bspline_w(float f, float w[3]) {

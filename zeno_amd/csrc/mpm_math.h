@@ -60,6 +60,9 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
 // (c, s) = (w, sigma a_pq) / sqrt(w^2 + a_pq^2): one reciprocal and two reciprocal roots.  (FP64
 // issue bounds the kernels that call it.  With this, no square root and divide in the strain and the
 // six entries of tau, two million sand particles: stress 127 -> 79 us, return mapping 141 -> 91.)
+// Against 80-bit arithmetic, 100,000 F with stretches within 5 % of 1 and within 1e-3 .. 1e3, RMS: |V L V^T -
+// A| / |A| 3.9e-16 and 3.7e-16 (with correctly rounded divides and roots 4.3e-16 and 4.1e-16), |V^T V - I|
+// 6.5e-16 and 6.0e-16 (7.2e-16 and 6.6e-16).
 __device__ __forceinline__ void jacobi_eig3(double A[3][3], double V[3][3]) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -175,6 +178,8 @@ __device__ __forceinline__ void polar_rotation(const double F[3][3], double R[3]
 // the singular values to 1 within 35 |E|^4 / 128 < 1e-16 in one step.  For F a few per cent from a
 // rotation that is two iterations and the series, where five iterations ran to a step of 1e-13.
 // (Stress of 800,000 fixed-corotated particles: 33.8 -> 19.3 us, of 4.9 million 169 -> 106.)
+// Error of R against 80-bit arithmetic, the same F: 1.0e-16 and 1.3e-16 RMS, 2.9e-16 and 4.8e-16 at most
+// (iterated to the end 1.6e-16 and 1.9e-16, 4.3e-16 and 6.0e-16).
 // For det F > 0 the polar factor is the rotation of the signed SVD, so this
 // agrees with polar_rotation to FP64 rounding.  Returns false (R untouched) if
 // det F is not clearly positive or the iteration has not converged in 16
